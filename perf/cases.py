@@ -265,8 +265,8 @@ def tolerance(case):
     # Seen against `exact`, and between launch tiles (other summation orders): grids and FP64 meshes
     # up to 6e-14 (residual norms), FP32 meshes up to 1.4e-6.
     if case["kind"] == "grid" or case["precision"] == 64:
-        return {"rel": 1e-11, "max": 1e-8}
-    return {"rel": 1e-5, "max": 1e-2}
+        return {"rel": 1e-11, "max": 1e-9}
+    return {"rel": 1e-5, "max": 1e-3}
 
 
 # -------------------------------------------------------------------------------------- exact --
