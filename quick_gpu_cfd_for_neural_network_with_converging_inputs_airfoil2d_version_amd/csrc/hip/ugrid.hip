@@ -89,6 +89,9 @@ struct Grid {
   size_t plane;        // mx * my
   const double* dx;    // mx widths (ghosts included)
   const double* dy;    // my
+  const double* rdx;   // recip() of every width
+  const double* rdy;
+  int plain;           // widths, gamma - 1 and reference Mach numbers are plain (see `recip`)
   const double* mco;   // ncase
   // State buffers: B[0] and B[1] alternate as accepted state and RK candidate, B[2] holds the
   // second RK stage; backward Euler rotates all three (accepted state, iterate, candidate).
@@ -134,12 +137,72 @@ struct Grid {
   Control* ctrl;
 };
 
-struct Prim {
-  double r, u, v, p;
+// A cell as its four faces see it: the primitives, and what both sides of every face would form
+// from them again.  x and y faces exchange the roles of u and v, which no derived value notices
+// (u^2 + v^2 is a commutative sum), and a reflection only negates a velocity.
+//   HLLC:    a = sqrt(gamma p / r), q = sqrt(r), E = p / (gamma - 1) + r (u^2 + v^2) / 2,
+//            H = (E + p) / r, e = E / r
+//   AUSM+-up: a, H = E + p, e = the reciprocal of r that quotients by r share
+struct Cell {
+  double r, u, v, p, a, q, E, H, e;
 };
 struct Flux {
   double m, x, y, e;  // mass, x momentum, y momentum, energy
 };
+
+// ---------------------------------------------------------------------------------------------
+// Quotients and square roots.  The kernels are bound by FP64 instruction issue, and most of it
+// was IEEE division (38 a cell) and square root (10): the compiler's division is 12 instructions,
+// of which seven (two range scalings, v_rcp_f64, two Newton steps) depend on the divisor alone.
+// Quotients with a common divisor therefore share those (`recip`), and inside a plain range the
+// scalings, which there multiply by one, are left out.  What is left are the compiler's own
+// operations in its order, so the bits are those of n / d and sqrt(x); outside the plain range
+// (PLAIN false) the compiler's division and square root are used.
+//
+// Plain (`plain_state`): density and pressure in (2^-100, 2^100), energy below 2^100, which bounds
+// the velocities through p > 0; cell widths, gamma - 1 and the reference Mach numbers likewise
+// (Grid::plain).  Every divisor the kernels form is then a normal number in (2^-400, 2^400).  A
+// numerator may be arbitrarily small where a velocity or a flux difference is (zero and rounding
+// noise ahead of a wave): such quotients are formed of the numerator times 2^200 (`quot_scaled`),
+// so that the remainder of the last step stays exact; the other small numerators are sums'
+// negligible terms.
+// ---------------------------------------------------------------------------------------------
+constexpr double kPlainLow = 0x1p-100, kPlainHigh = 0x1p100;
+constexpr double kScale = 0x1p200, kUnscale = 0x1p-200;
+
+__device__ __forceinline__ double recip(double d) {
+  double y = __builtin_amdgcn_rcp(d);
+  y = __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+  return __builtin_fma(y, __builtin_fma(-d, y, 1.0), y);
+}
+// n / d with y = recip(d).
+template <bool PLAIN>
+__device__ __forceinline__ double quot(double n, double d, double y) {
+  if (!PLAIN) return n / d;
+  const double q = n * y;
+  return __builtin_fma(__builtin_fma(-d, q, n), y, q);
+}
+template <bool PLAIN>
+__device__ __forceinline__ double quot(double n, double d) {
+  return quot<PLAIN>(n, d, PLAIN ? recip(d) : 0.0);
+}
+// 2^200 n / d for a numerator of any size.
+__device__ __forceinline__ double quot_scaled(double n, double d, double y) { return quot<true>(n * kScale, d, y); }
+template <bool PLAIN>
+__device__ __forceinline__ double root(double x) {
+  if (!PLAIN) return sqrt(x);
+  double h = __builtin_amdgcn_rsq(x);
+  double s = x * h;
+  h = h * 0.5;
+  const double e = __builtin_fma(-h, s, 0.5);
+  s = __builtin_fma(s, e, s);
+  h = __builtin_fma(h, e, h);
+  s = __builtin_fma(__builtin_fma(-s, s, x), h, s);
+  return __builtin_fma(__builtin_fma(-s, s, x), h, s);
+}
+__device__ __forceinline__ bool plain_state(double r, double p, double E) {
+  return r > kPlainLow && r < kPlainHigh && p > kPlainLow && E < kPlainHigh;
+}
 
 // ---------------------------------------------------------------------------------------------
 // Pointwise formulas (operation order of src/euler2d_cuda.cu:71-146, 169-205, 248-281).
@@ -148,52 +211,79 @@ __device__ __forceinline__ double pressure(double r, double mu, double mv, doubl
   return (gamma - 1.0) * (E - 0.5 * (mu * mu + mv * mv) / r);
 }
 
-__device__ __forceinline__ Prim primitive(double r, double mu, double mv, double E, double gamma) {
-  return {r, mu / r, mv / r, pressure(r, mu, mv, E, gamma)};
+// The primitives of a cell.  `ok` (PLAIN): whether its state is plain; the quotients hold only then.
+template <bool PLAIN>
+__device__ __forceinline__ Cell primitives(double r, double mu, double mv, double E, double gamma, double* y,
+                                           bool* ok) {
+  Cell c{};
+  c.r = r;
+  if (PLAIN) {
+    *y = recip(r);
+    c.p = (gamma - 1.0) * (E - quot<true>(0.5 * (mu * mu + mv * mv), r, *y));
+    *ok = plain_state(r, c.p, E);
+    c.u = __builtin_copysign(quot_scaled(mu, r, *y) * kUnscale, mu);  // r > 0; 0 / r keeps its sign
+    c.v = __builtin_copysign(quot_scaled(mv, r, *y) * kUnscale, mv);
+  } else {
+    *y = 0.0;
+    c.u = mu / r;
+    c.v = mv / r;
+    c.p = pressure(r, mu, mv, E, gamma);
+  }
+  return c;
 }
 
-// Exact flux along the normal velocity un (tangential ut): mass, normal, tangential, energy.
-__device__ __forceinline__ void exact_flux(double r, double un, double ut, double p, double gm, double f[4]) {
-  const double E = p / (gm - 1.0) + 0.5 * r * (un * un + ut * ut);
-  f[0] = r * un;
-  f[1] = r * un * un + p;
-  f[2] = r * un * ut;
-  f[3] = un * (E + p);
+// The derived values of a cell; y = recip(r) (PLAIN), yg = recip(gamma - 1).
+template <bool AUSM, bool PLAIN>
+__device__ __forceinline__ void derive(Cell& c, double gm, double y, double yg) {
+  c.a = root<PLAIN>(quot<PLAIN>(gm * c.p, c.r, y));
+  const double E = quot<PLAIN>(c.p, gm - 1.0, yg) + 0.5 * c.r * (c.u * c.u + c.v * c.v);
+  if (AUSM) {
+    c.H = E + c.p;
+    c.e = y;
+  } else {
+    c.q = root<PLAIN>(c.r);
+    c.E = E;
+    c.H = quot<PLAIN>(E + c.p, c.r, y);
+    c.e = quot<PLAIN>(E, c.r, y);
+  }
 }
 
-__device__ void hllc(double rL, double uL, double vL, double pL, double rR, double uR, double vR, double pR, double gm,
-                     double f[4]) {
-  const double aL = sqrt(gm * pL / rL), aR = sqrt(gm * pR / rR);
-  const double EL = pL / (gm - 1.0) + 0.5 * rL * (uL * uL + vL * vL);
-  const double ER = pR / (gm - 1.0) + 0.5 * rR * (uR * uR + vR * vR);
-  const double qL = sqrt(rL), qR = sqrt(rR);
-  const double HL = (EL + pL) / rL, HR = (ER + pR) / rR;
-  const double uT = (qL * uL + qR * uR) / (qL + qR);
-  const double vT = (qL * vL + qR * vR) / (qL + qR);
-  const double HT = (qL * HL + qR * HR) / (qL + qR);
-  const double aT = sqrt(fmax((gm - 1.0) * (HT - 0.5 * (uT * uT + vT * vT)), 1e-300));
-  const double SL = fmin(uL - aL, uT - aT), SR = fmax(uR + aR, uT + aT);
-  double fL[4], fR[4];
-  exact_flux(rL, uL, vL, pL, gm, fL);
-  exact_flux(rR, uR, vR, pR, gm, fR);
-  if (SL >= 0.0) {
-    for (int k = 0; k < 4; ++k) f[k] = fL[k];
-    return;
+// HLLC flux in the face frame; un, ut: the normal and tangential velocity of a side.
+template <bool PLAIN>
+__device__ __forceinline__ void hllc(const Cell& L, double uL, double vL, const Cell& R, double uR, double vR,
+                                     double gm, double f[4]) {
+  const double qs = L.q + R.q, ys = PLAIN ? recip(qs) : 0.0;
+  const double uT = quot<PLAIN>(L.q * uL + R.q * uR, qs, ys);
+  const double vT = quot<PLAIN>(L.q * vL + R.q * vR, qs, ys);
+  const double HT = quot<PLAIN>(L.q * L.H + R.q * R.H, qs, ys);
+  const double aT = root<PLAIN>(fmax((gm - 1.0) * (HT - 0.5 * (uT * uT + vT * vT)), 1e-300));
+  const double SL = fmin(uL - L.a, uT - aT), SR = fmax(uR + R.a, uT + aT);
+  // The side that the face's flux is built on: the upwind one outside the fan, that of the
+  // contact's sign inside it (where SL < 0 < SR).
+  bool left = SL >= 0.0;
+  const bool whole = left || SR <= 0.0;
+  const double dL = SL - uL, dR = SR - uR, mL = L.r * dL, mR = R.r * dR;
+  double Ss = 0.0;
+  if (!whole) {
+    Ss = quot<PLAIN>(R.p - L.p + L.r * uL * dL - R.r * uR * dR, mL - mR);
+    left = Ss >= 0.0;
   }
-  if (SR <= 0.0) {
-    for (int k = 0; k < 4; ++k) f[k] = fR[k];
-    return;
-  }
-  const double Ss = (pR - pL + rL * uL * (SL - uL) - rR * uR * (SR - uR)) / (rL * (SL - uL) - rR * (SR - uR));
-  // Star state of the upwind side of the contact, then F = F_side + S_side (U* - U_side).
-  const bool left = Ss >= 0.0;
-  const double r = left ? rL : rR, u = left ? uL : uR, v = left ? vL : vR, p = left ? pL : pR;
-  const double E = left ? EL : ER, S = left ? SL : SR;
-  const double* fs = left ? fL : fR;
-  const double a = r * (S - u) / (S - Ss);
-  const double star[4] = {a, a * Ss, a * v, a * (E / r + (Ss - u) * (Ss + p / (r * (S - u))))};
-  const double side[4] = {r, r * u, r * v, E};
-  for (int k = 0; k < 4; ++k) f[k] = fs[k] + S * (star[k] - side[k]);
+  const double r = left ? L.r : R.r, u = left ? uL : uR, v = left ? vL : vR, p = left ? L.p : R.p;
+  const double E = left ? L.E : R.E;
+  const double mass = r * u;
+  f[0] = mass;
+  f[1] = mass * u + p;
+  f[2] = mass * v;
+  f[3] = u * (E + p);
+  if (whole) return;
+  // Star state of that side, then F = F_side + S_side (U* - U_side).
+  const double S = left ? SL : SR, e = left ? L.e : R.e, m = left ? mL : mR;
+  const double a = quot<PLAIN>(m, S - Ss);
+  const double star = a * (e + (Ss - u) * (Ss + quot<PLAIN>(p, m)));
+  f[0] = f[0] + S * (a - r);
+  f[1] = f[1] + S * (a * Ss - mass);
+  f[2] = f[2] + S * (a * v - r * v);
+  f[3] = f[3] + S * (star - E);
 }
 
 // AUSM+-up split functions (Liou 2006) with the reference's constants (beta 1/8, Kp 1/4,
@@ -209,39 +299,39 @@ __device__ __forceinline__ double p5(double m, int s, double alpha) {
   return m2(m, s) * ((s * 2.0 - m) - s * 16.0 * alpha * m * m2(m, -s));
 }
 
-__device__ void ausm(double rL, double uL, double vL, double pL, double rR, double uR, double vR, double pR, double gm,
-                     double mco, double f[4]) {
-  const double a12 = 0.5 * (sqrt(gm * pL / rL) + sqrt(gm * pR / rR));
-  const double rho12 = 0.5 * (rL + rR), ML = uL / a12, MR = uR / a12;
-  const double mb2 = 0.5 * (uL * uL + uR * uR) / (a12 * a12);
+template <bool PLAIN>
+__device__ __forceinline__ void ausm(const Cell& L, double uL, double vL, const Cell& R, double uR, double vR,
+                                     double mco, double f[4]) {
+  const double a12 = 0.5 * (L.a + R.a), ya = PLAIN ? recip(a12) : 0.0;
+  const double rho12 = 0.5 * (L.r + R.r), ML = quot<PLAIN>(uL, a12, ya), MR = quot<PLAIN>(uR, a12, ya);
+  const double mb2 = quot<PLAIN>(0.5 * (uL * uL + uR * uR), a12 * a12);
   const double m02 = fmin(1.0, fmax(mb2, mco * mco));
-  const double fa = sqrt(m02) * (2.0 - sqrt(m02));
+  const double m0 = root<PLAIN>(m02);
+  const double fa = m0 * (2.0 - m0);
   const double alpha = 3.0 / 16.0 * (-4.0 + 5.0 * fa * fa);
-  const double m12 =
-      m4(ML, 1) + m4(MR, -1) - (0.25 / fa) * fmax(1.0 - mb2, 0.0) * (pR - pL) / (rho12 * a12 * a12);
+  const double m12 = m4(ML, 1) + m4(MR, -1) -
+                     quot<PLAIN>(quot<PLAIN>(0.25, fa) * fmax(1.0 - mb2, 0.0) * (R.p - L.p), rho12 * a12 * a12);
   const double pp = p5(ML, 1, alpha), pm = p5(MR, -1, alpha);
-  const double p12 = pp * pL + pm * pR - 0.75 * pp * pm * (rL + rR) * fa * a12 * (uR - uL);
+  const double p12 = pp * L.p + pm * R.p - 0.75 * pp * pm * (L.r + R.r) * fa * a12 * (uR - uL);
   const bool left = m12 > 0.0;
-  const double r = left ? rL : rR, u = left ? uL : uR;
-  const double v = left ? vL : vR, p = left ? pL : pR;
+  const double r = left ? L.r : R.r, u = left ? uL : uR, v = left ? vL : vR;
   const double mdot = a12 * m12 * r;
-  const double E = p / (gm - 1.0) + 0.5 * r * (u * u + v * v);
   f[0] = mdot;
   f[1] = mdot * u + p12;
   f[2] = mdot * v;
-  f[3] = mdot * (E + p) / r;
+  f[3] = quot<PLAIN>(mdot * (left ? L.H : R.H), r, left ? L.e : R.e);
 }
 
 // Flux through an x face (normal u) or a y face (normal v), returned in x / y momentum order.
-template <bool XFACE>
-__device__ __forceinline__ Flux face_flux(const Grid& g, double mco, const Prim& L, const Prim& R) {
+template <bool XFACE, bool AUSM, bool PLAIN>
+__device__ __forceinline__ Flux face_flux(double gamma, double mco, const Cell& L, const Cell& R) {
   double f[4];
   const double nL = XFACE ? L.u : L.v, tL = XFACE ? L.v : L.u;
   const double nR = XFACE ? R.u : R.v, tR = XFACE ? R.v : R.u;
-  if (g.ausm)
-    ausm(L.r, nL, tL, L.p, R.r, nR, tR, R.p, g.gamma, mco, f);
+  if (AUSM)
+    ausm<PLAIN>(L, nL, tL, R, nR, tR, mco, f);
   else
-    hllc(L.r, nL, tL, L.p, R.r, nR, tR, R.p, g.gamma, f);
+    hllc<PLAIN>(L, nL, tL, R, nR, tR, gamma, f);
   return XFACE ? Flux{f[0], f[1], f[2], f[3]} : Flux{f[0], f[2], f[1], f[3]};
 }
 
@@ -256,6 +346,24 @@ __device__ __forceinline__ double wave_bound(double r, double mu, double mv, dou
 __device__ __forceinline__ bool inadmissible(double r, double mu, double mv, double E, double gamma) {
   const double p = pressure(r, mu, mv, E, gamma);
   return !(r > 0.0) || !(p > 0.0) || !isfinite(r) || !isfinite(p);
+}
+
+// Admissibility of an RK candidate, and with WAVE its wave-speed bound: `inadmissible` and
+// `wave_bound` with the quotients by r shared (pressure and sound speed see the same p).
+template <bool WAVE>
+__device__ __forceinline__ bool check_candidate(double r, double mu, double mv, double E, const Grid& g, double dx,
+                                                double dy, double rdx, double rdy, double* bound) {
+  const double y = recip(r);
+  const double p = (g.gamma - 1.0) * (E - quot<true>(0.5 * (mu * mu + mv * mv), r, y));
+  if (__any(!(g.plain && plain_state(r, p, E)))) {
+    if (WAVE) *bound = wave_bound(r, mu, mv, E, g, dx, dy);
+    return inadmissible(r, mu, mv, E, g.gamma);
+  }
+  if (WAVE) {  // |u| and |v| are added to the sound speed: a tiny one's last bits vanish
+    const double a = root<true>(quot<true>(g.gamma * p, r, y));
+    *bound = quot<true>(fabs(quot<true>(mu, r, y)) + a, dx, rdx) + quot<true>(fabs(quot<true>(mv, r, y)) + a, dy, rdy);
+  }
+  return false;
 }
 
 // Ghost index map of one axis (src/euler2d_cuda.cu:153-180): the interior cell a ghost copies
@@ -396,8 +504,8 @@ __device__ void commit(const Grid& g) {
 // The cut-grid instantiation takes 140-144 VGPRs (3 waves per SIMD against the regular kernels'
 // 4); holding it to 4 waves spills 10-13 registers and was measured slower (2.40 against 2.37 ms
 // per step on 16 x 1024^2 with a body).
-template <int MODE, bool CUT>
-__global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __restrict__ rhs_in,
+template <int MODE, bool CUT, bool AUSM>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 3 : 4))) void k_stage(Grid g, const double* __restrict__ rhs_in,
                                                      double* __restrict__ rhs_out) {
   Control* ctrl = g.ctrl;
   bool skip = false;
@@ -421,7 +529,7 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
   constexpr double B = MODE == 2 ? 0.25 : MODE == 3 ? 2.0 / 3.0 : 1.0;
 
   const int lane = threadIdx.x % kLanes;
-  const int strip = logical_block() * kWaves + threadIdx.x / kLanes;
+  const int strip = __builtin_amdgcn_readfirstlane(logical_block() * kWaves + threadIdx.x / kLanes);
   bool wave_bad = false;
   unsigned long long bound = 0;
   const bool work = !skip && strip < g.strips;
@@ -439,10 +547,14 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
     const size_t plane = g.plane;
     const size_t case_base = static_cast<size_t>(icase) * 4 * plane + (ic + kGhosts);
     const double mco = g.mco[icase];
-    const double dxi = g.dx[min(max(i, -kGhosts), g.nx + kGhosts - 1) + kGhosts];
+    const int iw = min(max(i, -kGhosts), g.nx + kGhosts - 1) + kGhosts;
+    const double dxi = g.dx[iw], rdxi = g.rdx[iw];
+    const double yg = recip(g.gamma - 1.0);
     const double dt = MODE > 0 ? g.dt[icase] : 0.0;
 
-    Prim wprev{};
+    Cell wprev{};
+    // Whether the cells of the last three rows were evaluated by the plain quotients (bit 0: this row).
+    unsigned plain = 0u;
     Flux gprev{}, xres{};  // xres: x residual of a full cell, or ae FX_e - aw FX_w of a cut cell
     double ay_prev = 1.0;  // aperture of the previous y face (cut grids)
     double q0 = 0, q1 = 0, q2 = 0, q3 = 0;  // conserved state of the owned cell of the previous row
@@ -457,14 +569,24 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
       // (its faces, cut or not, rewritten by SRD or not).
       const unsigned code_m = CUT ? g.code[static_cast<size_t>(jc + kGhosts) * g.mx + ic + kGhosts] : 0u;
       const unsigned code_u = CUT && in_x ? g.code[static_cast<size_t>(j + kGhosts) * g.mx + i + kGhosts] : 0u;
-      Prim w;
-      if (CUT && (code_m & 1u)) {
-        w = Prim{1.0, 0.0, 0.0, 1.0};  // solid cell (never a ghost's source: the body keeps clear of the sides)
+      // A solid cell stands for (1, 0, 0, 1) (never a ghost's source: the body keeps clear of the sides).
+      const bool solid = CUT && (code_m & 1u);
+      double yr;
+      bool ok;
+      Cell w = primitives<true>(c0, c1, c2, c3, g.gamma, &yr, &ok);
+      if (solid) w.r = 1.0, w.u = 0.0, w.v = 0.0, w.p = 1.0, yr = 1.0, ok = true;
+      // (The residual alone, MODE 0, is asked for at states of any kind: always the general form.)
+      const bool plain_row = MODE != 0 && g.plain && !__any(!ok);
+      plain = (plain << 1 | (plain_row ? 1u : 0u)) & 7u;
+      if (plain_row) {
+        derive<AUSM, true>(w, g.gamma, yr, yg);
       } else {
-        w = primitive(c0, c1, c2, c3, g.gamma);
-        if (flip_u) w.u = -w.u;
-        if (flip_v) w.v = -w.v;
+        w = primitives<false>(c0, c1, c2, c3, g.gamma, &yr, &ok);
+        if (solid) w.r = 1.0, w.u = 0.0, w.v = 0.0, w.p = 1.0;
+        derive<AUSM, false>(w, g.gamma, 0.0, 0.0);
       }
+      if (flip_u) w.u = -w.u;
+      if (flip_v) w.v = -w.v;
       if (j >= j0) {
         // y face between rows j - 1 and j (closed faces carry no flux)
         double ay = 1.0;
@@ -473,10 +595,12 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
           ay = st == 0u ? 0.0 : st == 1u ? g.dx[i + kGhosts] : g.ayl[static_cast<size_t>(j) * g.nx + i];
         }
         Flux gf{0.0, 0.0, 0.0, 0.0};
-        if (!CUT || ay > 0.0) gf = face_flux<false>(g, mco, wprev, w);
+        if (!CUT || ay > 0.0)
+          gf = (plain & 3u) == 3u ? face_flux<false, AUSM, true>(g.gamma, mco, wprev, w)
+                                  : face_flux<false, AUSM, false>(g.gamma, mco, wprev, w);
         if (j > j0 && owner) {
           // Residual and update of the owned cell of row j - 1.
-          const double dyj = g.dy[j - 1 + kGhosts];
+          const double dyj = g.dy[j - 1 + kGhosts], rdyj = g.rdy[j - 1 + kGhosts];
           const size_t kc = static_cast<size_t>(j - 1 + kGhosts) * g.mx + i + kGhosts;
           double r0, r1, r2, r3;
           bool fluid = true, moved = false;
@@ -484,10 +608,17 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
             fluid = false;
             r0 = r1 = r2 = r3 = 0.0;
           } else if (!CUT || !(code_prev & 2u)) {
-            r0 = xres.m - (gf.m - gprev.m) / dyj;
-            r1 = xres.x - (gf.x - gprev.x) / dyj;
-            r2 = xres.y - (gf.y - gprev.y) / dyj;
-            r3 = xres.e - (gf.e - gprev.e) / dyj;
+            if (plain == 7u) {
+              r0 = __builtin_fma(-kUnscale, quot_scaled(gf.m - gprev.m, dyj, rdyj), xres.m);
+              r1 = __builtin_fma(-kUnscale, quot_scaled(gf.x - gprev.x, dyj, rdyj), xres.x);
+              r2 = __builtin_fma(-kUnscale, quot_scaled(gf.y - gprev.y, dyj, rdyj), xres.y);
+              r3 = __builtin_fma(-kUnscale, quot_scaled(gf.e - gprev.e, dyj, rdyj), xres.e);
+            } else {
+              r0 = xres.m - (gf.m - gprev.m) / dyj;
+              r1 = xres.x - (gf.x - gprev.x) / dyj;
+              r2 = xres.y - (gf.y - gprev.y) / dyj;
+              r3 = xres.e - (gf.e - gprev.e) / dyj;
+            }
           } else {
             const double iv = 1.0 / g.vol[kc], pw = wprev.p;
             r0 = -iv * (xres.m + ay * gf.m - ay_prev * gprev.m);
@@ -535,12 +666,14 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
             out[ko + plane] = n1;
             out[ko + 2 * plane] = n2;
             out[ko + 3 * plane] = n3;
-            if (fluid && inadmissible(n0, n1, n2, n3, g.gamma)) wave_bad = true;
-            // the next step's bound (cells that SRD rewrites report theirs after it)
-            if (MODE == 3 && fluid && !moved) {
-              const double b = wave_bound(n0, n1, n2, n3, g, dxi, dyj);
-              const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(b));
-              bound = bits > bound ? bits : bound;
+            if (fluid) {
+              double b = 0.0;
+              if (check_candidate<MODE == 3>(n0, n1, n2, n3, g, dxi, dyj, rdxi, rdyj, &b)) wave_bad = true;
+              // the next step's bound (cells that SRD rewrites report theirs after it)
+              if (MODE == 3 && !moved) {
+                const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(b));
+                bound = bits > bound ? bits : bound;
+              }
             }
           }
         }
@@ -549,23 +682,35 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
       }
       if (j >= j0 && j <= jl) {
         // x faces of row j: lane k evaluates the face west of its cell.
-        Prim wl;
+        // (Lane 0, which has no west neighbour, takes its own cell: __shfl_up returns it.)
+        Cell wl{};
         wl.r = shfl_up1(w.r);
         wl.u = shfl_up1(w.u);
         wl.v = shfl_up1(w.v);
         wl.p = shfl_up1(w.p);
-        if (lane == 0) wl = w;
+        wl.a = shfl_up1(w.a);
+        wl.H = shfl_up1(w.H);
+        wl.e = shfl_up1(w.e);
+        if (!AUSM) {
+          wl.q = shfl_up1(w.q);
+          wl.E = shfl_up1(w.E);
+        }
         double ax = 1.0;
         if (CUT && in_x) {
           const unsigned st = (code_u >> 3) & 3u;
           ax = st == 0u ? 0.0 : st == 1u ? g.dy[j + kGhosts] : g.axl[static_cast<size_t>(j) * (g.nx + 1) + i];
         }
         Flux fw{0.0, 0.0, 0.0, 0.0};
-        if (!CUT || ax > 0.0) fw = face_flux<true>(g, mco, wl, w);
+        if (!CUT || ax > 0.0)
+          fw = plain_row ? face_flux<true, AUSM, true>(g.gamma, mco, wl, w)
+                         : face_flux<true, AUSM, false>(g.gamma, mco, wl, w);
         const Flux fe{shfl_down1(fw.m), shfl_down1(fw.x), shfl_down1(fw.y), shfl_down1(fw.e)};
         const double ae = CUT ? shfl_down1(ax) : 1.0;
         if (CUT && owner && (code_u & 2u))
           xres = Flux{ae * fe.m - ax * fw.m, ae * fe.x - ax * fw.x, ae * fe.y - ax * fw.y, ae * fe.e - ax * fw.e};
+        else if (plain_row)
+          xres = Flux{-kUnscale * quot_scaled(fe.m - fw.m, dxi, rdxi), -kUnscale * quot_scaled(fe.x - fw.x, dxi, rdxi),
+                      -kUnscale * quot_scaled(fe.y - fw.y, dxi, rdxi), -kUnscale * quot_scaled(fe.e - fw.e, dxi, rdxi)};
         else
           xres = Flux{-(fe.m - fw.m) / dxi, -(fe.x - fw.x) / dxi, -(fe.y - fw.y) / dxi, -(fe.e - fw.e) / dxi};
       }
@@ -585,6 +730,11 @@ __global__ __launch_bounds__(kThreads) void k_stage(Grid g, const double* __rest
     bound = wave_max(bound);
     if (work && lane == 0 && bound) atomicMax(&g.smax[icase], bound);
   }
+}
+
+// recip() of the cell widths, once per session.
+__global__ void k_recip(const double* d, double* r, int n) {
+  for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) r[k] = recip(d[k]);
 }
 
 // The commit of a trial, one wave after the last stage (the kernel boundary orders every
@@ -946,6 +1096,7 @@ __global__ __launch_bounds__(kLanes) void k_be_check(Grid g) {
 // formulas in its order (so the same bits: neighbours are interior, the body keeps three cells
 // from every side), and raises the trial's flag if one is inadmissible; the stage kernels then
 // return at once.  The decision is the one the whole-grid pass would take.
+template <bool AUSM>
 __global__ __launch_bounds__(kThreads) void k_stage1_precheck(Grid g) {
   const Control* c = g.ctrl;
   if (__hip_atomic_load(&c->status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != RUNNING ||
@@ -962,20 +1113,24 @@ __global__ __launch_bounds__(kThreads) void k_stage1_precheck(Grid g) {
     const int jr = kc / g.mx - kGhosts, i = kc % g.mx - kGhosts;
     const double* u = in + icase * 4 * plane;
     const double mco = g.mco[icase], dt = g.dt[icase];
-    const auto prim_at = [&](int k) {
-      return g.vol[k] <= 0.0 ? Prim{1.0, 0.0, 0.0, 1.0}
-                             : primitive(u[k], u[k + plane], u[k + 2 * plane], u[k + 3 * plane], g.gamma);
+    const auto cell_at = [&](int k) {
+      double y;
+      bool ok;
+      Cell c = primitives<false>(u[k], u[k + plane], u[k + 2 * plane], u[k + 3 * plane], g.gamma, &y, &ok);
+      if (g.vol[k] <= 0.0) c.r = 1.0, c.u = 0.0, c.v = 0.0, c.p = 1.0;
+      derive<AUSM, false>(c, g.gamma, 0.0, 0.0);
+      return c;
     };
-    const Prim w = prim_at(kc);
+    const Cell w = cell_at(kc);
     const double ax = g.axl[static_cast<size_t>(jr) * (g.nx + 1) + i];
     const double ae = g.axl[static_cast<size_t>(jr) * (g.nx + 1) + i + 1];
     const double as = g.ayl[static_cast<size_t>(jr) * g.nx + i];
     const double an = g.ayl[static_cast<size_t>(jr + 1) * g.nx + i];
     Flux fw{0.0, 0.0, 0.0, 0.0}, fe{0.0, 0.0, 0.0, 0.0}, gs{0.0, 0.0, 0.0, 0.0}, gn{0.0, 0.0, 0.0, 0.0};
-    if (ax > 0.0) fw = face_flux<true>(g, mco, prim_at(kc - 1), w);
-    if (ae > 0.0) fe = face_flux<true>(g, mco, w, prim_at(kc + 1));
-    if (as > 0.0) gs = face_flux<false>(g, mco, prim_at(kc - g.mx), w);
-    if (an > 0.0) gn = face_flux<false>(g, mco, w, prim_at(kc + g.mx));
+    if (ax > 0.0) fw = face_flux<true, AUSM, false>(g.gamma, mco, cell_at(kc - 1), w);
+    if (ae > 0.0) fe = face_flux<true, AUSM, false>(g.gamma, mco, w, cell_at(kc + 1));
+    if (as > 0.0) gs = face_flux<false, AUSM, false>(g.gamma, mco, cell_at(kc - g.mx), w);
+    if (an > 0.0) gn = face_flux<false, AUSM, false>(g.gamma, mco, w, cell_at(kc + g.mx));
     const Flux xres{ae * fe.m - ax * fw.m, ae * fe.x - ax * fw.x, ae * fe.y - ax * fw.y, ae * fe.e - ax * fw.e};
     const double iv = 1.0 / g.vol[kc], pw = w.p;
     const double r0 = -iv * (xres.m + an * gn.m - as * gs.m);
@@ -1204,10 +1359,15 @@ int grid_blocks(const Grid& g, size_t items) {
 // A stage kernel in the regular or the cut-grid instantiation.
 template <int MODE>
 void launch_stage(ugrid_session* s, hipStream_t stream, const double* in = nullptr, double* out = nullptr) {
-  if (s->g.has_cut)
-    hipLaunchKernelGGL((k_stage<MODE, true>), dim3(s->launch_blocks), dim3(kThreads), 0, stream, s->g, in, out);
+  const dim3 blocks(s->launch_blocks), threads(kThreads);
+  if (s->g.has_cut && s->g.ausm)
+    hipLaunchKernelGGL((k_stage<MODE, true, true>), blocks, threads, 0, stream, s->g, in, out);
+  else if (s->g.has_cut)
+    hipLaunchKernelGGL((k_stage<MODE, true, false>), blocks, threads, 0, stream, s->g, in, out);
+  else if (s->g.ausm)
+    hipLaunchKernelGGL((k_stage<MODE, false, true>), blocks, threads, 0, stream, s->g, in, out);
   else
-    hipLaunchKernelGGL((k_stage<MODE, false>), dim3(s->launch_blocks), dim3(kThreads), 0, stream, s->g, in, out);
+    hipLaunchKernelGGL((k_stage<MODE, false, false>), blocks, threads, 0, stream, s->g, in, out);
 }
 
 // A stage kernel followed, on a cut grid with small cells, by the redistribution of its candidate.
@@ -1219,7 +1379,10 @@ void launch_stage_srd(ugrid_session* s, hipStream_t stream) {
     // the trial's commit (the stage kernels then return at once).
     const dim3 pre_blocks(grid_blocks(g, static_cast<size_t>(g.ncase) * g.n_pre));
     for (int r = 0; r < kPrechecks; ++r) {
-      hipLaunchKernelGGL(k_stage1_precheck, pre_blocks, dim3(kThreads), 0, stream, g);
+      if (g.ausm)
+        hipLaunchKernelGGL(k_stage1_precheck<true>, pre_blocks, dim3(kThreads), 0, stream, g);
+      else
+        hipLaunchKernelGGL(k_stage1_precheck<false>, pre_blocks, dim3(kThreads), 0, stream, g);
       if (r + 1 < kPrechecks) hipLaunchKernelGGL(k_precheck_reject, dim3(1), dim3(kLanes), 0, stream, g);
     }
   }
@@ -1501,7 +1664,14 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   if (dt)
     for (int c = 0; c < g.ncase; ++c) dt0[c] = dt[c];
 
-  double *dxd = nullptr, *dyd = nullptr, *mcod = nullptr;
+  const auto plain_value = [](double x) { return x > kPlainLow && x < kPlainHigh; };
+  bool plain = plain_value(p.gamma - 1.0) && plain_value(p.gamma);
+  for (int k = 0; k < g.mx; ++k) plain = plain && plain_value(setup->dx[k]);
+  for (int k = 0; k < g.my; ++k) plain = plain && plain_value(setup->dy[k]);
+  for (int c = 0; c < g.ncase; ++c) plain = plain && plain_value(mco[c]);
+  g.plain = plain ? 1 : 0;
+
+  double *dxd = nullptr, *dyd = nullptr, *rdx = nullptr, *rdy = nullptr, *mcod = nullptr;
   if (!ok(hipGetDevice(&s->device), err, err_len, "hipGetDevice") ||
       !ok(hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking), err, err_len, "hipStreamCreate") ||
       !ok(hipHostMalloc(reinterpret_cast<void**>(&s->host_ctrl), sizeof(Control), hipHostMallocDefault), err, err_len,
@@ -1510,7 +1680,8 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
       !device_alloc(s, &g.B[2], states, err, err_len) || !device_alloc(s, &dxd, g.mx, err, err_len) ||
       (p.time_integrator == 1 && !device_alloc(s, &g.R, states, err, err_len)) ||
       !device_alloc(s, &g.norm, g.ncase, err, err_len) || !device_alloc(s, &g.initial, g.ncase, err, err_len) ||
-      !device_alloc(s, &dyd, g.my, err, err_len) || !device_alloc(s, &mcod, g.ncase, err, err_len) ||
+      !device_alloc(s, &dyd, g.my, err, err_len) || !device_alloc(s, &rdx, g.mx, err, err_len) ||
+      !device_alloc(s, &rdy, g.my, err, err_len) || !device_alloc(s, &mcod, g.ncase, err, err_len) ||
       !device_alloc(s, &g.t, g.ncase, err, err_len) || !device_alloc(s, &g.dt, g.ncase, err, err_len) ||
       !device_alloc(s, &g.dt_out, g.ncase, err, err_len) || !device_alloc(s, &g.smax, g.ncase, err, err_len) ||
       !device_alloc(s, &g.ctrl, 1, err, err_len)) {
@@ -1519,6 +1690,8 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   }
   g.dx = dxd;
   g.dy = dyd;
+  g.rdx = rdx;
+  g.rdy = rdy;
   g.mco = mcod;
   Control c0{};
   c0.status = 0;
@@ -1540,6 +1713,12 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
       !ok(hipMemsetAsync(g.smax, 0, g.ncase * sizeof(unsigned long long), s->stream), err, err_len, "clear bound") ||
       !ok(hipMemcpyAsync(g.ctrl, &c0, sizeof(Control), h2d, s->stream), err, err_len, "upload control") ||
       !ok(hipStreamSynchronize(s->stream), err, err_len, "upload")) {
+    release(s);
+    return 3;
+  }
+  hipLaunchKernelGGL(k_recip, dim3(grid_blocks(g, g.mx)), dim3(kThreads), 0, s->stream, dxd, rdx, g.mx);
+  hipLaunchKernelGGL(k_recip, dim3(grid_blocks(g, g.my)), dim3(kThreads), 0, s->stream, dyd, rdy, g.my);
+  if (!ok(hipGetLastError(), err, err_len, "cell widths")) {
     release(s);
     return 3;
   }

@@ -1,0 +1,78 @@
+"""The grid kernels' shared quotients (plain range), their general form outside it, and the two
+ways the strips report their maxima: bitwise the oracle at states that sit on the borders.
+
+The oracle divides and takes roots in IEEE arithmetic.  Inside the plain range (density and
+pressure within 2^+-100) the kernels' quotients are the compiler's division without its range
+scalings; velocities may be of any size, down to subnormal numbers, and of either zero sign.
+Outside it a row falls back to full divisions, so both must give the oracle's bits (results that
+are themselves subnormal excepted: nothing here makes one).
+"""
+import numpy as np
+import pytest
+
+from oracle import pygrid as G
+from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import euler2d as E
+
+pytestmark = pytest.mark.gpu
+
+
+def solver(nx, ny, cases, flux, scale=1.0, velocity=0.3, mco=0.7, seed=5):
+    """Random states: density about 1, pressure about `scale`, velocities `velocity` times the
+    sound speed; one half of the first case has velocities of exactly +0 / -0."""
+    par = E.params2d_default()
+    par.limiter, par.flux = E.LIM_FIRST_ORDER, flux
+    s = E.Solver2D(nx, ny, 0.0, 1.0, 0.0, 0.7, cases, par)
+    rng = np.random.default_rng(seed)
+    for c in range(cases):
+        r = rng.uniform(0.5, 2.0, (ny, nx))
+        p = scale * rng.uniform(0.5, 2.0, (ny, nx))
+        u, v = (velocity * np.sqrt(scale) * rng.uniform(-1, 1, (ny, nx)) for _ in range(2))
+        if c == 0:
+            u[: ny // 2], v[: ny // 2] = 0.0, -0.0
+        s.set_primitive_field(c, r, u, v, p)
+        s.set_mco(c, mco)
+    return s
+
+
+def check(s, steps):
+    ref = G.run(s, 1e300, steps)
+    with s.device_session() as d:
+        status, message = d.run(1e300, steps)
+        d.pull()
+    assert status == ref["status"], message
+    assert (s.nsteps, s.nreject) == (ref["nsteps"], ref["nreject"])
+    for got, want in ((s.U, ref["u"]), (s.t, ref["t"]), (s.dt, ref["dt"])):
+        np.testing.assert_array_equal(got, want)
+
+
+@pytest.mark.parametrize("flux", [E.FLUX_HLLC, E.FLUX_AUSMPUP])
+@pytest.mark.parametrize("scale, velocity", [
+    (1.0, 0.3), (1.0, 3.0),          # plain
+    (1.0, 1e-120), (1.0, 1e-290),    # plain, with velocities whose products underflow
+    (2.0 ** -99, 0.3), (2.0 ** 98, 0.3),    # the last plain pressures: some cells on either side
+    (2.0 ** -140, 0.3), (2.0 ** 140, 0.3),  # general
+])
+def test_states_at_the_borders_of_the_plain_range(flux, scale, velocity):
+    check(solver(70, 9, 2, flux, scale, velocity), 6)
+
+
+@pytest.mark.parametrize("flux", [E.FLUX_HLLC, E.FLUX_AUSMPUP])
+def test_one_odd_row_among_plain_ones(flux):
+    s = solver(130, 12, 1, flux)
+    q = s.field(0)
+    q[3, 7, 40] = 2.0 ** 101  # energy beyond the plain range in one cell: its row takes the general form
+    check(s, 3)
+
+
+def test_reference_mach_number_outside_the_plain_range():
+    check(solver(64, 8, 2, E.FLUX_AUSMPUP, mco=2.0 ** -120), 4)
+
+
+@pytest.mark.parametrize("cases", [1023, 1025])  # strips' partials in the decision kernel's table / atomics
+def test_many_cases(cases):
+    check(solver(3, 4, cases, E.FLUX_HLLC), 5)
+
+
+@pytest.mark.parametrize("nx, ny, cases", [(1, 1, 1), (62, 1, 3), (63, 65, 1), (124, 130, 2), (500, 77, 5)])
+def test_strip_lengths(nx, ny, cases):
+    check(solver(nx, ny, cases, E.FLUX_HLLC), 4)
