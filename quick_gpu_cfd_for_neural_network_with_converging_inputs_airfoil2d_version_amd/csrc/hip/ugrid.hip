@@ -501,11 +501,18 @@ __device__ void commit(const Grid& g) {
 //   MODE 4: R = L(Q), per case max over cells of max_v |dt R - (Q - U)| / max(1, |U|)
 //           (infinite for a non-finite defect), src/euler2d_cuda.cu:331-350
 // ---------------------------------------------------------------------------------------------
-// The cut-grid instantiation takes 140-144 VGPRs (3 waves per SIMD against the regular kernels'
-// 4); holding it to 4 waves spills 10-13 registers and was measured slower (2.40 against 2.37 ms
-// per step on 16 x 1024^2 with a body).
+__device__ __forceinline__ void load_row(const double* p, size_t plane, double (&c)[4]) {
+  for (int v = 0; v < 4; ++v) c[v] = p[v * plane];
+}
+// Bound by FP64 instruction issue (about 480 VALU instructions a cell, 930 with every quotient a full
+// division and both sides' sound speeds, energies and enthalpies formed at every face) and by the
+// latency of its row's loads: the next row's state is loaded while this one is evaluated, the base
+// state of the row to update before the y fluxes.  That takes 136 VGPRs (150-160 on a cut grid) and
+// three waves per SIMD; four waves (128 VGPRs) spill nothing but the loads' lead: 8 cases of
+// 1024 x 1024, HLLC, stages 336 / 347 / 378 us before, 218 / 276 / 294 with four waves and no
+// prefetch, 202 / 230 / 244 with it.
 template <int MODE, bool CUT, bool AUSM>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 3 : 4))) void k_stage(Grid g, const double* __restrict__ rhs_in,
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 2 : 3))) void k_stage(Grid g, const double* __restrict__ rhs_in,
                                                      double* __restrict__ rhs_out) {
   Control* ctrl = g.ctrl;
   bool skip = false;
@@ -560,14 +567,25 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
     double q0 = 0, q1 = 0, q2 = 0, q3 = 0;  // conserved state of the owned cell of the previous row
     unsigned code_prev = 0;                  // cut grids: code of the lane's cell of the previous row
     const bool in_x = i >= 0 && i <= g.nx;   // the lane's west x face is a grid face
+    bool flip_v = false, flip_next = false;
+    int jc = map_axis(j0 - 1, g.ny, g.bc[2], g.bc[3], &flip_v);
+    double next[4];
+    load_row(in + case_base + static_cast<size_t>(jc + kGhosts) * g.mx, plane, next);
     for (int j = j0 - 1; j <= jl + 1; ++j) {
-      bool flip_v = false;
-      const int jc = map_axis(j, g.ny, g.bc[2], g.bc[3], &flip_v);
-      const size_t k = case_base + static_cast<size_t>(jc + kGhosts) * g.mx;
-      const double c0 = in[k], c1 = in[k + plane], c2 = in[k + 2 * plane], c3 = in[k + 3 * plane];
+      const double c0 = next[0], c1 = next[1], c2 = next[2], c3 = next[3];
+      const size_t ko = case_base + static_cast<size_t>(j - 1 + kGhosts) * g.mx;
+      const int jm = jc; const bool flip_m = flip_v;
+      if (j <= jl) {
+        flip_v = false;
+        jc = map_axis(j + 1, g.ny, g.bc[2], g.bc[3], &flip_v);
+        load_row(in + case_base + static_cast<size_t>(jc + kGhosts) * g.mx, plane, next);
+      }
+      double base_row[4];
+      if (MODE > 1 && MODE < 4 && j > j0 && owner)
+        for (int v = 0; v < 4; ++v) base_row[v] = __builtin_nontemporal_load(base + ko + v * plane);
       // Cut grids: codes of the mapped cell (solid or not) and of the lane's own column at row j
       // (its faces, cut or not, rewritten by SRD or not).
-      const unsigned code_m = CUT ? g.code[static_cast<size_t>(jc + kGhosts) * g.mx + ic + kGhosts] : 0u;
+      const unsigned code_m = CUT ? g.code[static_cast<size_t>(jm + kGhosts) * g.mx + ic + kGhosts] : 0u;
       const unsigned code_u = CUT && in_x ? g.code[static_cast<size_t>(j + kGhosts) * g.mx + i + kGhosts] : 0u;
       // A solid cell stands for (1, 0, 0, 1) (never a ghost's source: the body keeps clear of the sides).
       const bool solid = CUT && (code_m & 1u);
@@ -586,7 +604,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
         derive<AUSM, false>(w, g.gamma, 0.0, 0.0);
       }
       if (flip_u) w.u = -w.u;
-      if (flip_v) w.v = -w.v;
+      if (flip_m) w.v = -w.v;
       if (j >= j0) {
         // y face between rows j - 1 and j (closed faces carry no flux)
         double ay = 1.0;
@@ -629,7 +647,6 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
             r2 -= iv * pw * g.way[kc];
           }
           if (CUT && MODE == 3) moved = (code_prev & 4u) != 0u;
-          const size_t ko = case_base + static_cast<size_t>(j - 1 + kGhosts) * g.mx;
           if (MODE == 0 || MODE == 4) {
             out[ko] = r0;
             out[ko + plane] = r1;
@@ -653,10 +670,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
           } else {
             double a0 = q0, a1 = q1, a2 = q2, a3 = q3;
             if (MODE > 1) {
-              a0 = __builtin_nontemporal_load(base + ko);
-              a1 = __builtin_nontemporal_load(base + ko + plane);
-              a2 = __builtin_nontemporal_load(base + ko + 2 * plane);
-              a3 = __builtin_nontemporal_load(base + ko + 3 * plane);
+              a0 = base_row[0], a1 = base_row[1], a2 = base_row[2], a3 = base_row[3];
             }
             const double n0 = A * a0 + B * (q0 + dt * r0);
             const double n1 = A * a1 + B * (q1 + dt * r1);
