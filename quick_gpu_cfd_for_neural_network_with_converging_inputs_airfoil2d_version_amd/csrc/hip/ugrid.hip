@@ -48,6 +48,12 @@ constexpr int kThreads = kLanes * kWaves;
 constexpr int kGhosts = 2;
 constexpr int kXcds = 8;
 constexpr int kMaxRetries = 12;
+constexpr int kDecide = 1024;      // threads of the decision kernels that reduce the strips' partials
+// Cases up to which strips store their maxima for the decision kernel instead of one 64-bit
+// atomicMax per strip on the case's word: device-scope atomics on one word take about 9 ns each
+// (4 cases of 400 x 311, 2184 strips: last stage 44 us, of which 20 us were its atomics).  With more
+// cases the words are many and the reduction's table would not fit LDS.
+constexpr int kPartCases = 1024;
 // First-stage pre-checks per trial on a cut grid (the body bench needs about six halvings a step).
 constexpr int kPrechecks = 8;
 enum : int { BC_PERIODIC = 0, BC_TRANSMISSIVE = 1, BC_REFLECT = 2 };
@@ -101,6 +107,11 @@ struct Grid {
   double* dt;          // step of the running trial
   double* dt_out;      // last accepted step
   unsigned long long* smax;  // per case: bit pattern of the largest wave-speed bound (non-negative)
+  // Per strip: the largest bound (last RK stage) or scaled defect (backward Euler) of its cells, which
+  // the one-block decision kernel reduces per case.  With more than kPartCases cases the strips
+  // report to smax / norm by atomics instead.
+  unsigned long long* part;
+  int use_part;
   unsigned long long* norm;  // per case: bit pattern of the largest scaled defect (backward Euler)
   double* initial;           // per case: first defect norm of the physical step
   double pseudo0, rtol, atol;
@@ -451,20 +462,43 @@ __device__ void reject(const Grid& g) {
   }
 }
 
-__device__ void commit(const Grid& g) {
+// Maxima of the strips' partials per case, in LDS (one block, all threads).
+__device__ void reduce_parts(const Grid& g, unsigned long long* s_max) {
+  const int tid = threadIdx.x, lane = tid % kLanes;
+  for (int k = tid; k < g.ncase; k += blockDim.x) s_max[k] = 0;
+  __syncthreads();
+  const int per_case = g.strips_x * g.strips_y;
+  for (int first = tid - lane; first < g.strips; first += blockDim.x) {
+    const int strip = first + lane;
+    const bool valid = strip < g.strips;
+    const unsigned long long v = valid ? g.part[strip] : 0ull;
+    const int c = (valid ? strip : g.strips - 1) / per_case;
+    if (__all(c == __shfl(c, 0, kLanes))) {
+      const unsigned long long m = wave_max(v);
+      if (lane == 0) atomicMax(&s_max[c], m);
+    } else if (valid) {
+      atomicMax(&s_max[c], v);
+    }
+  }
+  __syncthreads();
+}
+
+__device__ void commit(const Grid& g, unsigned long long* s_max) {
   Control* c = g.ctrl;
-  const int lane = threadIdx.x % kLanes;
+  const int tid = threadIdx.x;
   if (__hip_atomic_load(&c->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) {
-    reject(g);
+    __syncthreads();  // every wave has read the flag that reject() clears
+    if (tid < kLanes) reject(g);
     return;
   }
+  if (g.use_part) reduce_parts(g, s_max);
   // Accepted: advance the clocks of the cases that moved, then either stop (maxsteps reached,
   // or every case at tend) or choose the next step from the candidate's wave-speed bound.
   const double tend = c->tend;
   const long long steps = c->steps + 1;
   const bool maxed = steps >= c->maxsteps;
   int open = 0;
-  for (int k = lane; k < g.ncase; k += kLanes) {
+  for (int k = tid; k < g.ncase; k += blockDim.x) {
     const double d = g.dt[k];
     g.dt_out[k] = d;
     double tk = g.t[k];
@@ -474,12 +508,15 @@ __device__ void commit(const Grid& g) {
     }
     if (tk < tend) open = 1;
   }
-  const bool next = !maxed && __any(open);
-  for (int k = lane; k < g.ncase; k += kLanes) {
-    if (next) g.dt[k] = next_dt(g, __longlong_as_double(static_cast<long long>(load_relaxed(&g.smax[k]))), g.t[k], tend);
+  const bool any_open = __syncthreads_or(open);
+  const bool next = !maxed && any_open;
+  for (int k = tid; k < g.ncase; k += blockDim.x) {
+    unsigned long long m = load_relaxed(&g.smax[k]);
+    if (g.use_part) m = s_max[k] > m ? s_max[k] : m;
+    if (next) g.dt[k] = next_dt(g, __longlong_as_double(static_cast<long long>(m)), g.t[k], tend);
     g.smax[k] = 0;
   }
-  if (lane == 0) {
+  if (tid == 0) {
     c->steps = steps;
     c->cur ^= 1;
     c->nsteps += 1;
@@ -736,13 +773,23 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
   if (MODE == 0) return;
   if (MODE == 4) {
     bound = wave_max(bound);
-    if (work && lane == 0 && bound) atomicMax(&g.norm[icase], bound);
+    if (work && lane == 0) {
+      if (g.use_part)
+        g.part[strip] = bound;
+      else if (bound)
+        atomicMax(&g.norm[icase], bound);
+    }
     return;
   }
   if (__any(wave_bad) && lane == 0) atomicOr(&ctrl->bad, 1);
   if (MODE == 3) {
     bound = wave_max(bound);
-    if (work && lane == 0 && bound) atomicMax(&g.smax[icase], bound);
+    if (work && lane == 0) {
+      if (g.use_part)
+        g.part[strip] = bound;
+      else if (bound)
+        atomicMax(&g.smax[icase], bound);
+    }
   }
 }
 
@@ -751,12 +798,14 @@ __global__ void k_recip(const double* d, double* r, int n) {
   for (int k = blockIdx.x * blockDim.x + threadIdx.x; k < n; k += gridDim.x * blockDim.x) r[k] = recip(d[k]);
 }
 
-// The commit of a trial, one wave after the last stage (the kernel boundary orders every
+// The commit of a trial, one block after the last stage (the kernel boundary orders every
 // stage's flags and bounds before it; an in-kernel last-arriver commit would need device-scope
 // fences, which write back and invalidate an XCD's L2 and cost more than this launch).
-__global__ __launch_bounds__(kLanes) void k_commit(Grid g) {
+__global__ __launch_bounds__(kDecide) void k_commit(Grid g) {
+  __shared__ unsigned long long s_max[kPartCases];
+  // (The status moves only after the block's first barrier.)
   if (g.ctrl->status != RUNNING) return;
-  commit(g);
+  commit(g, s_max);
 }
 
 // Wave-speed bound of every case at U[cur] (the first step of a run, src/euler2d_cuda.cu:223-237).
@@ -959,13 +1008,18 @@ __global__ __launch_bounds__(kThreads) void k_be_copy(Grid g) {
 // step's first norm) per case; on convergence the iterate becomes the accepted state and the
 // clocks advance (implicit2d_advance_time), else a candidate follows or the iteration limit
 // ends the run with 4.
-__global__ __launch_bounds__(kLanes) void k_be_decide(Grid g) {
+__global__ __launch_bounds__(kDecide) void k_be_decide(Grid g) {
+  __shared__ unsigned long long s_max[kPartCases];
   Control* c = g.ctrl;
   if (c->status != RUNNING || (c->phase != PH_COPY && c->phase != PH_RES)) return;
+  __syncthreads();  // every wave has read the phase that the first one moves
+  if (g.use_part) reduce_parts(g, s_max);
+  if (threadIdx.x >= kLanes) return;
+  const unsigned long long* norms = g.use_part ? s_max : g.norm;
   const int lane = threadIdx.x;
   int nonfinite = 0;
   for (int k = lane; k < g.ncase; k += kLanes)
-    if (!isfinite(__longlong_as_double(static_cast<long long>(g.norm[k])))) nonfinite = 1;
+    if (!isfinite(__longlong_as_double(static_cast<long long>(norms[k])))) nonfinite = 1;
   if (__any(nonfinite)) {
     for (int k = lane; k < g.ncase; k += kLanes) g.norm[k] = 0;
     if (lane == 0) {
@@ -979,7 +1033,7 @@ __global__ __launch_bounds__(kLanes) void k_be_decide(Grid g) {
   unsigned long long imax = 0, nmax = 0, tmax = 0;
   int open = 0;
   for (int k = lane; k < g.ncase; k += kLanes) {
-    const double norm = __longlong_as_double(static_cast<long long>(g.norm[k]));
+    const double norm = __longlong_as_double(static_cast<long long>(norms[k]));
     if (first) g.initial[k] = norm;
     const double initial = g.initial[k];
     const double tol = fmax(g.atol, g.rtol * initial);
@@ -1419,7 +1473,7 @@ int launch_be_round(ugrid_session* s, hipStream_t stream) {
   hipLaunchKernelGGL(k_be_open, dim3(1), dim3(kLanes), 0, stream, g);
   hipLaunchKernelGGL(k_be_copy, dim3(grid_blocks(g, 4 * cells)), dim3(kThreads), 0, stream, g);
   launch_stage<4>(s, stream);
-  hipLaunchKernelGGL(k_be_decide, dim3(1), dim3(kLanes), 0, stream, g);
+  hipLaunchKernelGGL(k_be_decide, dim3(1), dim3(kDecide), 0, stream, g);
   hipLaunchKernelGGL(k_be_trial, dim3(grid_blocks(g, cells)), dim3(kThreads), 0, stream, g);
   hipLaunchKernelGGL(k_be_check, dim3(1), dim3(kLanes), 0, stream, g);
   return 7;
@@ -1429,7 +1483,7 @@ int launch_trial(ugrid_session* s, hipStream_t stream) {
   launch_stage_srd<1>(s, stream);
   launch_stage_srd<2>(s, stream);
   launch_stage_srd<3>(s, stream);
-  hipLaunchKernelGGL(k_commit, dim3(1), dim3(kLanes), 0, stream, s->g);
+  hipLaunchKernelGGL(k_commit, dim3(1), dim3(kDecide), 0, stream, s->g);
   return 4;
 }
 
@@ -1667,6 +1721,7 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   }
   g.strips = static_cast<int>(strips);
   g.blocks = (g.strips + kWaves - 1) / kWaves;
+  g.use_part = g.ncase <= kPartCases ? 1 : 0;
   s->launch_blocks = (g.blocks + kXcds - 1) / kXcds * kXcds;
 
   std::vector<double> mco(g.ncase, p.ausm_mco);
@@ -1693,7 +1748,8 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
       !device_alloc(s, &g.B[0], states, err, err_len) || !device_alloc(s, &g.B[1], states, err, err_len) ||
       !device_alloc(s, &g.B[2], states, err, err_len) || !device_alloc(s, &dxd, g.mx, err, err_len) ||
       (p.time_integrator == 1 && !device_alloc(s, &g.R, states, err, err_len)) ||
-      !device_alloc(s, &g.norm, g.ncase, err, err_len) || !device_alloc(s, &g.initial, g.ncase, err, err_len) ||
+      !device_alloc(s, &g.norm, g.ncase, err, err_len) ||
+      !device_alloc(s, &g.part, g.use_part ? g.strips : 1, err, err_len) || !device_alloc(s, &g.initial, g.ncase, err, err_len) ||
       !device_alloc(s, &dyd, g.my, err, err_len) || !device_alloc(s, &rdx, g.mx, err, err_len) ||
       !device_alloc(s, &rdy, g.my, err, err_len) || !device_alloc(s, &mcod, g.ncase, err, err_len) ||
       !device_alloc(s, &g.t, g.ncase, err, err_len) || !device_alloc(s, &g.dt, g.ncase, err, err_len) ||
@@ -1920,7 +1976,7 @@ extern "C" int ugrid_profile(ugrid_session* s, int32_t trials, double* stage_us,
     (void)hipEventRecord(e[2], s->stream);
     launch_stage_srd<3>(s, s->stream);
     (void)hipEventRecord(e[3], s->stream);
-    hipLaunchKernelGGL(k_commit, dim3(1), dim3(kLanes), 0, s->stream, g);
+    hipLaunchKernelGGL(k_commit, dim3(1), dim3(kDecide), 0, s->stream, g);
   }
   good = good && ok(hipGetLastError(), err, err_len, "profile launch") &&
          ok(hipStreamSynchronize(s->stream), err, err_len, "profile");
