@@ -1626,13 +1626,29 @@ bool upload_cut(ugrid_session* s, const ugrid_cut_view& c, const double* dx, con
   return true;
 }
 
-// Rows per strip: 32, halved (down to 4) while the launch would hold fewer than 16 waves per
-// CU (256 CUs), and never more than the grid has.
-int choose_rows(int nx, int ny, int ncase) {
+// Rows per strip.  A strip of r rows costs its wave about r + 1 row times (the halo row's
+// primitives and y flux), and a CU that holds n = 1, 2, 3 blocks (three is what the registers admit)
+// takes kRowTime[n] microseconds a row, as fitted to launches of 1 to 64 rows on five grids.  Long
+// strips waste least on the halo, short ones spread a small grid over the chip, and a launch that
+// leaves its last round of blocks nearly empty pays for a whole one: the count with the least estimate
+// is chosen.  Against 32 rows, halved down to 4 while a CU held fewer than 16 waves: 8 cases of
+// 1024 x 1024 682 us a step at 32 rows and 594 at 47 (2992 waves of 3072 slots), 3 of 200 x 131
+// 39.4 us at 4 rows and 27.6 at 1, 4 of 400 x 311 70.6 us at 4 and 62.3 at 3.
+int choose_rows(int nx, int ny, int ncase, bool cut) {
+  constexpr int kCus = 256, kResident = 3, kLongest = 64;
+  constexpr double kRowTime[2][kResident + 1] = {{0.0, 1.95, 2.8, 3.6}, {0.0, 3.1, 4.1, 5.0}};
+  const double* row_time = kRowTime[cut ? 1 : 0];
   const long long sx = (nx + kStripCells - 1) / kStripCells;
-  int rows = 32;
-  while (rows > 4 && sx * ((ny + rows - 1) / rows) * ncase < 16LL * 256) rows /= 2;
-  return rows < ny ? rows : ny;
+  int best = 1;
+  double least = HUGE_VAL;
+  for (int rows = 1; rows <= std::min(kLongest, ny); ++rows) {
+    const long long strips = sx * ((ny + rows - 1) / rows) * ncase;
+    const long long blocks = (strips + kWaves - 1) / kWaves, per_cu = (blocks + kCus - 1) / kCus;
+    const double cost = (rows + 1) * (static_cast<double>(per_cu / kResident) * row_time[kResident] +
+                                      row_time[per_cu % kResident]);
+    if (cost < least) least = cost, best = rows;
+  }
+  return best;
 }
 
 }  // namespace
@@ -1711,7 +1727,7 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   g.rtol = p.implicit_rtol;
   g.atol = p.implicit_atol;
   g.maxiter = p.implicit_maxiter;
-  g.rows = choose_rows(g.nx, g.ny, g.ncase);
+  g.rows = choose_rows(g.nx, g.ny, g.ncase, setup->cut != nullptr);
   g.strips_x = (g.nx + kStripCells - 1) / kStripCells;
   g.strips_y = (g.ny + g.rows - 1) / g.rows;
   const long long strips = static_cast<long long>(g.strips_x) * g.strips_y * g.ncase;
