@@ -38,7 +38,11 @@ HIP_SOURCES = ["hip/amr_kernels_f64.hip", "hip/amr_kernels_f32.hip", "hip/amr_de
 # 1e-38; the FP64 state, control and reductions keep full IEEE behaviour.
 # The tensor-product grid solver is compiled without FMA contraction: its arithmetic follows the
 # reference's formulas operation for operation, so results are bitwise its CPU restatement's.
-HIP_EXTRA = {"hip/amr_kernels_f32.hip": ["-fno-hip-fp32-correctly-rounded-divide-sqrt", "-fgpu-flush-denormals-to-zero"],
+# The time-step kernels contract multiplies and adds within an expression only: which of them fuse
+# is then fixed by the source, and the instantiations of a kernel (launch shapes) give the same bits.
+HIP_EXTRA = {"hip/amr_kernels_f64.hip": ["-ffp-contract=on"],
+             "hip/amr_kernels_f32.hip": ["-ffp-contract=on", "-fno-hip-fp32-correctly-rounded-divide-sqrt",
+                                         "-fgpu-flush-denormals-to-zero"],
              "hip/ugrid.hip": ["-ffp-contract=off"]}
 INCLUDES = ["-I", str(ROOT / "include"), "-I", str(CSRC / "host"), "-I", str(CSRC / "hip")]
 ARCH = os.environ.get("HIPAMR_ARCH", "gfx950")

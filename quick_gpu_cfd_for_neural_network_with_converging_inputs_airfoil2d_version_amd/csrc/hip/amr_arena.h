@@ -102,7 +102,7 @@ struct MeshDesc {
 template <class T>
 struct ArenaPtrs {
   int n_meshes, nc, nf, nw, tile;
-  // Threads per cell of the flux launches (1 or 2; tile * flux_spread <= 256): the face items of
+  // Threads per cell of the flux launches (1 to 3; tile * flux_spread <= 512): the face items of
   // a tile are spread over flux_spread * tile threads, the cell work stays on the first tile.
   int flux_spread;
   int n_cell_blocks, n_face_blocks, n_wall_blocks;

@@ -280,6 +280,7 @@ int capture_all(amr_batch* b, char* err, size_t err_len) {
 // Stream, pinned control mirrors, optional graph; the arena is already built.
 int finish_setup(amr_batch* b, Clock::time_point t0, char* err, size_t err_len) {
   const int n = b->n;
+  b->spread = b->arena->flux_spread();
   if (!checked(hipHostMalloc(reinterpret_cast<void**>(&b->host_control), n * sizeof(Control), hipHostMallocDefault),
                err, err_len, "AMR pinned control") ||
       !checked(hipHostMalloc(reinterpret_cast<void**>(&b->host_targets), n * sizeof(double), hipHostMallocDefault), err,

@@ -66,8 +66,9 @@ class Arena {
   // Base primitives of every running slot whose host-written state has none yet; follows every
   // launch_target before trials are launched.
   virtual int launch_prims(hipStream_t s) = 0;
-  // Threads per cell of the flux launches (1 or 2, at most 256 threads per block); launches
-  // issued after the call use it.  False: not a valid spread at this tile.
+  // Threads per cell of the flux launches (1 to 3, at most 512 threads per block); launches
+  // issued after the call use it.  False: not a valid spread at this tile.  An arena starts with the
+  // spread that its size calls for.
   virtual bool set_flux_spread(int spread) = 0;
   virtual int flux_spread() const = 0;
   // Independent branches of the trial (slots m with m % n_branches() == j) and the trial of one

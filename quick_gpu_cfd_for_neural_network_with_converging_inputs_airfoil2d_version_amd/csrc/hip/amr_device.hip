@@ -80,6 +80,22 @@ bool tables_ready(const amr_mesh_view& v) {
 }
 
 inline int round_up(int n, int tile) { return (n + tile - 1) / tile * tile; }
+
+// Threads per cell of the flux launches of an arena of `tiles` tiles: the most (up to three, one
+// face item each) at which all its waves are resident at once.  Such a launch is bound by its
+// blocks' latency, of which the rounds of face items are the largest part; beyond that the second
+// half of the kernel, which one thread per cell does, idles registers that other blocks need.
+// Trials of one mesh at 1 / 2 / 3 threads per cell: LF2 FP64 69 / 62 / 56 us, FP32 57 / 53 / 47;
+// level 7 FP64 77 / 70 / 64; level 8 FP64 (1640 tiles, over the line at 2) 124 / 128 / 132, FP32
+// 97 / 93 / 90.  8 LF2 meshes at tile 128, FP32, 73 / 67 / 64; 16 of mixed levels 103 / 101 / 117 and
+// FP64 176 / 210 / 273.
+int flux_spread_for(int tiles, int tile, int precision) {
+  const int resident = 256 * 4 * (precision == 64 ? 2 : 7);  // waves that the flux kernels' registers admit
+  int spread = 3;
+  while (spread > 1 && (tile * spread > 512 || static_cast<long long>(tiles) * (tile / 64) * spread > resident))
+    --spread;
+  return spread;
+}
 inline size_t align256(size_t b) { return (b + 255) / 256 * 256; }
 
 // Element counts of an arena's index spaces.
@@ -867,7 +883,7 @@ class DeviceArena final : public Arena {
     a.nf = nf;
     a.nw = nw;
     a.tile = tile_;
-    a.flux_spread = 1;
+    a.flux_spread = flux_spread_for(n_cell_blocks_, tile_, sizeof(T) == 8 ? 64 : 32);
     a.n_cell_blocks = n_cell_blocks_;
     a.n_grid_blocks = table_offsets_[1];  // the whole-arena table
     a.commit_first = 0;
@@ -981,7 +997,7 @@ class DeviceArena final : public Arena {
   }
   int launch_prims(hipStream_t s) override { return hipamr::launch_prims<T>(ptrs_, s, nullptr); }
   bool set_flux_spread(int spread) override {
-    if ((spread != 1 && spread != 2) || tile_ * spread > 256) return false;  // launch bound
+    if (spread < 1 || spread > 3 || tile_ * spread > 512) return false;  // launch bound
     ptrs_.flux_spread = spread;
     return true;
   }

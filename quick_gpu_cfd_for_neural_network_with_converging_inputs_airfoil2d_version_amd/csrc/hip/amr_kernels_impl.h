@@ -36,6 +36,7 @@ namespace hipamr {
 namespace {
 
 constexpr int kMaxTile = 256;
+constexpr int kMaxThreads = 512;  // threads of the largest block (a flux launch of several threads per cell)
 constexpr unsigned long long kInfBits = 0x7ff0000000000000ull;
 
 enum : int { PASS_BASE = 0, PASS_STAGE = 1 };
@@ -320,7 +321,7 @@ __device__ __forceinline__ bool make_prim(const double* u, int nc, int k, const 
 // Minimum over the block of a double (wave64 xor-shuffles, then one LDS slot per wave).
 // All threads of the block must call it; the result is valid in thread 0.
 __device__ __forceinline__ double block_min(double v) {
-  __shared__ double part[kMaxTile / 64];
+  __shared__ double part[kMaxThreads / 64];
   for (int off = 32; off > 0; off >>= 1) v = fmin(v, __shfl_xor(v, off, 64));
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   if (lane == 0) part[wave] = v;
@@ -801,11 +802,14 @@ __device__ __forceinline__ void arrive_and_commit(Control* c, int n_blocks, bool
 // (72 VGPRs, 4 and 6 spilled; LDS for 14 blocks per CU).
 // On 256 LF2 meshes: base flux 187 -> 177 us, stage flux 188 -> 181 us against the unbounded
 // kernels; 8 waves (64 VGPRs) spills 11-14 and is slower.  FP64 (190-200 VGPRs) has no bound.
-// SPREAD threads per cell (1 or 2): a tile's face items are spread over SPREAD * tile threads,
+// SPREAD threads per cell (1 to 3): a tile's face items are spread over SPREAD * tile threads,
 // the cell work stays on the first tile of them (a separate instantiation, so that the one-thread
-// kernel keeps its registers).
+// kernel keeps its registers).  A tile touches 2.2 - 2.7 faces per cell, so three threads per cell
+// evaluate them in one round instead of three in a row: what a launch too small to fill the chip
+// takes is its blocks' latency (see flux_spread_for).
 template <class T, int STAGE, int SPREAD>
-__global__ __launch_bounds__(kMaxTile) __attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (STAGE == 0 ? 5 : 7) : 1)))
+__global__ __launch_bounds__(SPREAD == 1 ? kMaxTile : kMaxThreads)
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (STAGE == 0 ? 5 : 7) : 1)))
 void k_flux(ArenaPtrs<T> a) {
   constexpr bool BASE = STAGE == 0;
   const int2 blk = cell_block(a);
@@ -1346,7 +1350,9 @@ inline int blocks_of(int n, int tile) { return (n + tile - 1) / tile; }
 #define HIPAMR_LAUNCH_FLUX(name, STAGE, grid, lds, ...)                                                   \
   do {                                                                                                   \
     if (hook) hook->before(name);                                                                        \
-    if (a.flux_spread == 2)                                                                              \
+    if (a.flux_spread == 3)                                                                              \
+      hipLaunchKernelGGL((k_flux<T, STAGE, 3>), grid, dim3(3 * a.tile), lds, s, __VA_ARGS__);          \
+    else if (a.flux_spread == 2)                                                                         \
       hipLaunchKernelGGL((k_flux<T, STAGE, 2>), grid, dim3(2 * a.tile), lds, s, __VA_ARGS__);          \
     else                                                                                                 \
       hipLaunchKernelGGL((k_flux<T, STAGE, 1>), grid, dim3(a.tile), lds, s, __VA_ARGS__);              \
