@@ -20,22 +20,39 @@
 
 namespace hipamr {
 
-struct Control {
+struct alignas(128) Control {
   double time, target, dt;   // dt: step size of the last trial (halved on rejection)
   double trial_dt;           // step size of the running trial
-  unsigned long long dt_min; // bit pattern of the minimum local dt of the base pass
   long long steps, rejected, maxsteps;
   int bad, fatal, retrying, attempt, finished, active;
   int cur;                   // buffer holding the accepted state: U[cur]
   int w_valid;               // W/PHI hold primitives of U[cur]
   int r0_valid;              // R0 holds L(U[cur]) (set after a rejection)
   int wbuf;                  // primitive-vector buffer (0..2) holding the primitives of U[cur]
-  // Blocks of the last stage pass that have finished this trial (low 32 bits) and how many of
-  // them found the candidate inadmissible (high 32 bits); the last one commits (zero between
-  // trials).
+  // Gather lines whose blocks have all finished this trial, as GatherLine::arrivals; the block that
+  // completes the last one commits.
   unsigned long long arrivals;
 };
-static_assert(sizeof(Control) == 112, "Control layout");
+static_assert(sizeof(Control) == 128, "Control layout");
+
+// Where the blocks of a slot report their smallest local dt and their arrival at the end of a trial:
+// kGatherLines lines per slot, each a cache line of its own, of which a slot of at most kOneLineTiles
+// tiles uses the first and a larger one all, tile t line t % kGatherLines.  Device atomics on one word
+// take about 9 ns each and hold up reads of their cache line, so in the control records, 112 bytes
+// apart, they delayed every block of the slot and its neighbours: one level-8 mesh (1640 tiles) 124 ->
+// 98 us a trial in FP64 and 90 -> 62 in FP32, 16 meshes of mixed levels 99 -> 91, 8 LF2 meshes at
+// tile 64 71 -> 64.  One LF2 mesh (150 tiles) would lose 0.8 us to the second round of atomics.
+struct GatherLine {
+  unsigned long long dt_min;    // bit pattern of the minimum local dt of the base pass
+  // Blocks of the last stage pass that have finished this trial (low 32 bits) and how many of
+  // them found the candidate inadmissible (high 32 bits); zero between trials.
+  unsigned long long arrivals;
+  unsigned long long pad[14];
+};
+static_assert(sizeof(GatherLine) == 128, "GatherLine layout");
+constexpr int kGatherLines = 32;
+constexpr int kOneLineTiles = 160;
+__host__ __device__ constexpr int gather_lines(int tiles) { return tiles <= kOneLineTiles ? 1 : kGatherLines; }
 
 enum : int { VISC_VOLUME = 0, VISC_SRD_RATE = 1, VISC_SRD_GROUP = 2 };
 
@@ -114,6 +131,7 @@ struct ArenaPtrs {
   int commit_in_flux;
   const MeshDesc<T>* desc;
   Control* ctrl;
+  GatherLine* gather;          // kGatherLines per slot (gather_lines(n_tiles) in use)
   const int2* block_rec;       // n_grid_blocks: {tile, slot} of each block of a cell launch, {-1, -1} none
   const int* face_block_mesh;  // n_face_blocks + n_wall_blocks (faces first, then walls)
   // cells
@@ -207,7 +225,7 @@ template <class T>
 void launch_monitor(const ArenaPtrs<T>& a, hipStream_t stream);
 // Set the target time and step cap of every mesh and start a trial.  targets/maxsteps are
 // device arrays of n_meshes entries, or null to use the scalar values for all meshes.
-void launch_target(Control* ctrl, int n_meshes, double target, long long maxsteps, const double* targets,
+void launch_target(Control* ctrl, GatherLine* gather, int n_meshes, double target, long long maxsteps, const double* targets,
                    const long long* maxsteps_each, hipStream_t stream);
 
 }  // namespace hipamr

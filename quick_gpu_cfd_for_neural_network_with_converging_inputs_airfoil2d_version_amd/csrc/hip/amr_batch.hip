@@ -3,7 +3,7 @@
 // One arena of slots.  With two or more slots the trial runs as independent branches (slot m in
 // branch m % branches), each captured as its own graph and replayed on its own stream, so that
 // one branch's kernels fill the GPU while another's drain; the streams join at every poll.  The
-// host polls the array of control records (112 bytes per slot) every batch_trials trials; in
+// host polls the array of control records (128 bytes per slot) every batch_trials trials; in
 // amr_batch_advance the polls are pipelined through two pinned snapshots (queue_batch).  Slot
 // independence: every kernel reads only its own slot's ranges and control record, the only cross-block
 // reductions (minimum dt, monitor partials) are per slot and exact (atomicMin on the bit
@@ -447,7 +447,7 @@ int amr_batch_set_targets(amr_batch* b, const double* targets, const int64_t* ma
                               hipMemcpyHostToDevice, b->stream),
                err, err_len, "AMR step caps H2D"))
     return 1;
-  hipamr::launch_target(b->arena->control(), b->n, 0.0, 0, b->arena->target_array(), b->arena->maxsteps_array(),
+  hipamr::launch_target(b->arena->control(), b->arena->gather_lines(), b->n, 0.0, 0, b->arena->target_array(), b->arena->maxsteps_array(),
                         b->stream);
   b->arena->launch_prims(b->stream);  // base primitives of slots whose state the host wrote
   if (!checked(hipGetLastError(), err, err_len, "AMR target kernel")) return 1;
@@ -597,7 +597,6 @@ int amr_batch_monitor(amr_batch* b, const int32_t* mask, const double* frames, c
     if (use[m]) {
       e.bad = 0;
       e.r0_valid = 0;
-      e.dt_min = hipamr::kInfBitsHost;
     }
   }
   for (int m = 0; m < n; ++m) {
@@ -626,7 +625,6 @@ int amr_batch_monitor(amr_batch* b, const int32_t* mask, const double* frames, c
     const bool bad = b->host_control[m].bad || b->host_control[m].fatal;
     restore[m].w_valid = bad ? 0 : 1;
     restore[m].r0_valid = 0;
-    restore[m].dt_min = hipamr::kInfBitsHost;
     if (bad) {
       status[m] = 1;
       continue;

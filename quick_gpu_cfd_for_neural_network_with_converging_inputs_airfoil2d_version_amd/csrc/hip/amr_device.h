@@ -76,6 +76,7 @@ class Arena {
   virtual int n_branches() const = 0;
   virtual int launch_trial_branch(int j, hipStream_t s) = 0;
   virtual Control* control() = 0;
+  virtual GatherLine* gather_lines() = 0;
   // Device arrays of per-slot targets / step caps used by launch_target.
   virtual double* target_array() = 0;
   virtual long long* maxsteps_array() = 0;

@@ -195,7 +195,7 @@ SlabPlan plan_slab(const Totals& t, int nv) {
                arr(4, t.groups) + arr(sizeof(T), t.groups) + arr(4, t.members) + arr(8, t.cell_blocks) +
                2 * arr(4, t.walls) + 4 * arr(sizeof(T), t.walls) + 2 * arr(8, t.walls);
   p.control = arr(sizeof(Control), t.meshes) + arr(sizeof(double), t.meshes) + arr(sizeof(long long), t.meshes) +
-              arr(6 * sizeof(double), t.meshes);
+              arr(6 * sizeof(double), t.meshes) + arr(sizeof(GatherLine) * kGatherLines, t.meshes);
   p.cplane = arr(sizeof(T), t.cells);
   p.dplane = arr(sizeof(double), t.cells);
   p.vec4 = arr(4 * sizeof(T), t.cells);
@@ -849,6 +849,8 @@ class DeviceArena final : public Arena {
     frames_ = reinterpret_cast<double*>(base + offset);
     a.mon_frame = frames_;
     offset += align256(nm * 6 * sizeof(double));
+    a.gather = reinterpret_cast<GatherLine*>(base + offset);
+    offset += align256(nm * kGatherLines * sizeof(GatherLine));
     const size_t tables_end = offset;
     const auto dplanes = [&](int count) {
       double* p = reinterpret_cast<double*>(base + offset);
@@ -1003,6 +1005,7 @@ class DeviceArena final : public Arena {
   }
   int flux_spread() const override { return ptrs_.flux_spread; }
   Control* control() override { return ptrs_.ctrl; }
+  GatherLine* gather_lines() override { return ptrs_.gather; }
   double* target_array() override { return targets_; }
   long long* maxsteps_array() override { return maxsteps_; }
   hipError_t launch_monitor(hipStream_t s, const double* frames) override {
@@ -1078,7 +1081,6 @@ class DeviceArena final : public Arena {
     c.steps = meta.steps;
     c.rejected = meta.rejected;
     c.finished = 1;
-    c.dt_min = kInf;
     return c;
   }
 

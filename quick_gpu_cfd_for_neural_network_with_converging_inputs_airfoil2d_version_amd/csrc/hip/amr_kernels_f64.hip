@@ -4,9 +4,9 @@
 
 namespace hipamr {
 
-void launch_target(Control* ctrl, int n, double target, long long maxsteps, const double* targets,
+void launch_target(Control* ctrl, GatherLine* gather, int n, double target, long long maxsteps, const double* targets,
                    const long long* maxsteps_each, hipStream_t s) {
-  hipLaunchKernelGGL(k_target, dim3(blocks_of(n, 256)), dim3(256), 0, s, ctrl, n, target, maxsteps, targets,
+  hipLaunchKernelGGL(k_target, dim3(blocks_of(n, 256)), dim3(256), 0, s, ctrl, gather, n, target, maxsteps, targets,
                      maxsteps_each);
 }
 

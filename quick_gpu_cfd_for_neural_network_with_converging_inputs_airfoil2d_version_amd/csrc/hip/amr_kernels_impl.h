@@ -332,9 +332,29 @@ __device__ __forceinline__ double block_min(double v) {
   return r;
 }
 
-__device__ __forceinline__ void publish_dt(Control* c, double local) {
+// The gather line of a tile.
+template <class T>
+__device__ __forceinline__ GatherLine* gather_line(const ArenaPtrs<T>& a, const MeshDesc<T>& d, int m, int tile) {
+  return a.gather + static_cast<size_t>(m) * kGatherLines + (tile - d.first_cell_block) % gather_lines(d.n_tiles);
+}
+
+__device__ __forceinline__ void publish_dt(GatherLine* line, double local) {
   const double m = block_min(local);
-  if (threadIdx.x == 0 && m < INFINITY) atomicMin(&c->dt_min, static_cast<unsigned long long>(__double_as_longlong(m)));
+  if (threadIdx.x == 0 && m < INFINITY)
+    atomicMin(&line->dt_min, static_cast<unsigned long long>(__double_as_longlong(m)));
+}
+
+// The smallest local dt of the slot (every lane of the wave).
+template <class T>
+__device__ __forceinline__ unsigned long long gathered_dt(const ArenaPtrs<T>& a, const MeshDesc<T>& d, int m) {
+  const int lines = gather_lines(d.n_tiles);
+  unsigned long long v = a.gather[static_cast<size_t>(m) * kGatherLines + threadIdx.x % lines].dt_min;
+  if (lines == 1) return v;
+  for (int off = kGatherLines / 2; off > 0; off >>= 1) {
+    const unsigned long long o = __shfl_xor(v, off, 64);
+    v = o < v ? o : v;
+  }
+  return v;
 }
 
 // ------------------------------------------------------------------------------------------
@@ -360,8 +380,8 @@ __global__ __launch_bounds__(kMaxTile) void k_base_prim(ArenaPtrs<T> a) {
 
 // ------------------------------------------------------------------------------------------
 // Step size of the trial (reference choose_dt_kernel semantics, src/static_amr2d_cuda.cu:177-187).
-__device__ __forceinline__ bool choose_dt(const Control* c, double fixed, double* dt_out) {
-  double dt = c->retrying ? c->dt : (fixed > 0 ? fixed : __longlong_as_double(static_cast<long long>(c->dt_min)));
+__device__ __forceinline__ bool choose_dt(const Control* c, double fixed, unsigned long long dt_min, double* dt_out) {
+  double dt = c->retrying ? c->dt : (fixed > 0 ? fixed : __longlong_as_double(static_cast<long long>(dt_min)));
   const double remaining = c->target - c->time;
   dt = fmin(dt, remaining);
   const double tol = 32 * DBL_EPSILON * fmax(fmax(fabs(c->target), fabs(c->time)), dt);
@@ -374,13 +394,14 @@ __device__ __forceinline__ bool choose_dt(const Control* c, double fixed, double
 // same control fields; the slot's first block records the trial step or the fatal code (2: the
 // base residual failed, 4: dt underflow).  False: no stage this trial.
 template <class T>
-__device__ __forceinline__ bool open_stage0(Control* c, const MeshDesc<T>& d, int tile, double* dt) {
+__device__ __forceinline__ bool open_stage0(Control* c, const MeshDesc<T>& d, int tile, unsigned long long dt_min,
+                                            double* dt) {
   const bool leader = tile == d.first_cell_block && threadIdx.x == 0;
   if (c->bad & BAD_BASE) {  // the base residual failed: nonphysical base state
     if (leader) c->fatal = 2;
     return false;
   }
-  if (!choose_dt(c, d.dt_fixed, dt)) {
+  if (!choose_dt(c, d.dt_fixed, dt_min, dt)) {
     if (leader) c->fatal = 4;
     return false;
   }
@@ -746,7 +767,6 @@ __device__ __forceinline__ void begin_trial(Control* c) {
   }
   c->bad = 0;
   c->active = 1;
-  if (!c->r0_valid) c->dt_min = kInfBits;
 }
 
 // Accept or reject the finished trial of a slot (reference commit_control_kernel,
@@ -779,18 +799,26 @@ __device__ __forceinline__ void commit_trial(Control* c, bool bad) {
   begin_trial(c);
 }
 
+// Counts a block (low word) and whether it failed (high word); true, with whether any block failed,
+// in the block that completes the count, which clears it.
+__device__ __forceinline__ bool last_arrival(unsigned long long* count, int n_blocks, bool* failed) {
+  const unsigned long long before = atomicAdd(count, 1ull | (*failed ? (1ull << 32) : 0ull));
+  if (static_cast<int>(before & 0xffffffffull) + 1 != n_blocks) return false;
+  *failed = *failed || (before >> 32) != 0;
+  *count = 0;
+  return true;
+}
+
 // A block of the last stage pass has finished (`failed`: some thread of it found the candidate
-// inadmissible).  One 64-bit atomic per block counts the blocks (low word) and the failed ones
-// (high word); the block that completes the count commits the trial and clears the count.  Every
-// other block has made its last access to the slot's data and control by then, and the flags
-// raised in earlier launches are visible, so the commit needs no memory fence.
-__device__ __forceinline__ void arrive_and_commit(Control* c, int n_blocks, bool failed) {
-  const unsigned long long add = 1ull | (failed ? (1ull << 32) : 0ull);
-  const unsigned long long before = atomicAdd(&c->arrivals, add);
-  if (static_cast<int>(before & 0xffffffffull) + 1 != n_blocks) return;
-  const bool any_failed = (before >> 32) != 0 || failed;
-  c->arrivals = 0;
-  commit_trial(c, c->bad != 0 || any_failed);
+// inadmissible).  One 64-bit atomic per block counts the blocks of its gather line, and one per line the
+// lines; the block that completes the count commits the trial.  Every other block has made
+// its last access to the slot's data and control by then, and the flags raised in earlier launches
+// are visible, so the commit needs no memory fence.  `index`: the block's tile within the slot.
+__device__ __forceinline__ void arrive_and_commit(Control* c, GatherLine* line, int n_blocks, int index, bool failed) {
+  const int lines = gather_lines(n_blocks), g = index % lines;
+  if (!last_arrival(&line->arrivals, (n_blocks - g + lines - 1) / lines, &failed)) return;
+  if (lines > 1 && !last_arrival(&c->arrivals, lines, &failed)) return;
+  commit_trial(c, c->bad != 0 || failed);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1095,10 +1123,14 @@ void k_flux(ArenaPtrs<T> a) {
     }
   }
   }  // !failed
-  if (BASE && d.visc_mode != VISC_SRD_GROUP) publish_dt(c, local_dt);
+  GatherLine* const line = BASE || commits ? gather_line(a, d, m, tile) : nullptr;
+  if (BASE && d.visc_mode != VISC_SRD_GROUP) publish_dt(line, local_dt);
+  // The gathered steps have been read (by the launch before): the next base pass starts from none.
+  if (STAGE == 1 && tile == d.first_cell_block && tid < gather_lines(d.n_tiles))
+    a.gather[static_cast<size_t>(m) * kGatherLines + tid].dt_min = kInfBits;
   if (commits) {
     const int any = __syncthreads_or(bad);
-    if (tid == 0) arrive_and_commit(c, d.n_tiles, any != 0);
+    if (tid == 0) arrive_and_commit(c, line, d.n_tiles, tile - d.first_cell_block, any != 0);
   } else if (bad) {
     flag_bad(c, bad);
   }
@@ -1143,7 +1175,7 @@ __global__ __launch_bounds__(kMaxTile) void k_dt_group(ArenaPtrs<T> a) {
     if (rate > T(0)) dt = fmin(dt, d.transport.viscous_cfl / rate);
     local = static_cast<double>(dt);
   }
-  publish_dt(c, local);
+  publish_dt(gather_line(a, d, m, tile), local);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1162,7 +1194,7 @@ __global__ __launch_bounds__(kMaxTile) void k_stage0(ArenaPtrs<T> a) {
   if (!running(c)) return;
   const MeshDesc<T>& d = a.desc[m];
   double dt;
-  if (!open_stage0(c, d, tile, &dt)) return;
+  if (!open_stage0(c, d, tile, gathered_dt(a, d, m), &dt)) return;
   const int k = tile * static_cast<int>(blockDim.x) + static_cast<int>(threadIdx.x);
   if (k >= d.cell_begin + d.n_cells) return;
   // U1 = U + D1, D1 = T(dt R0) not stored (the next stage re-forms it); or U1 in U[cur ^ 1].
@@ -1246,7 +1278,7 @@ __global__ void k_commit(Control* ctrl, int n, int first, int stride) {
   commit_trial(c, c->bad != 0);
 }
 
-__global__ void k_target(Control* ctrl, int n, double target, long long maxsteps, const double* targets,
+__global__ void k_target(Control* ctrl, GatherLine* gather, int n, double target, long long maxsteps, const double* targets,
                          const long long* maxsteps_each) {
   const int m = static_cast<int>(blockIdx.x * blockDim.x + threadIdx.x);
   if (m >= n) return;
@@ -1255,6 +1287,10 @@ __global__ void k_target(Control* ctrl, int n, double target, long long maxsteps
   c->maxsteps = maxsteps_each ? maxsteps_each[m] : maxsteps;
   c->finished = c->time >= c->target;
   begin_trial(c);
+  for (int g = 0; g < kGatherLines; ++g) {
+    gather[static_cast<size_t>(m) * kGatherLines + g].arrivals = 0;
+    gather[static_cast<size_t>(m) * kGatherLines + g].dt_min = kInfBits;
+  }
 }
 
 // Sum over the block of several doubles (same wave64 + LDS pattern as block_min); valid in thread 0.

@@ -2,7 +2,7 @@
 //
 // Semantics follow the reference backend (src/static_amr2d_cuda.cu:219-366): create validates,
 // uploads and captures one trial as a graph; advance replays it batch_trials times per host
-// poll of the 112-byte control record until the target time is reached (0), a fatal code is
+// poll of the 128-byte control record until the target time is reached (0), a fatal code is
 // raised (1, last accepted state retained) or the wall budget expires (2); download copies
 // the accepted state; stats reports the same counters as AmrGpuStats.
 #include <algorithm>
@@ -174,7 +174,7 @@ int amr_hip_advance(amr_session* s, double tend, int64_t maxsteps, double wall_b
   const auto t0 = Clock::now();
   auto last = t0;
   bool expired = false;
-  hipamr::launch_target(s->arena->control(), 1, tend, maxsteps, nullptr, nullptr, s->stream);
+  hipamr::launch_target(s->arena->control(), s->arena->gather_lines(), 1, tend, maxsteps, nullptr, nullptr, s->stream);
   s->arena->launch_prims(s->stream);  // base primitives when the state was written by the host
   for (;;) {
     if (s->options.event_timing && !checked(hipEventRecord(s->start, s->stream), err, err_len, "AMR timing record start"))
@@ -263,7 +263,6 @@ int amr_hip_rhs(amr_session* s, const double* u, uint64_t u_len, double* r, char
   eval.bad = 0;
   eval.w_valid = 0;
   eval.r0_valid = 0;
-  eval.dt_min = 0x7ff0000000000000ull;
   Control after{};
   if (!checked(copy_sync(s->arena->control(), &eval, sizeof(Control), hipMemcpyHostToDevice, s->stream), err, err_len,
                "AMR control H2D") ||
@@ -279,7 +278,6 @@ int amr_hip_rhs(amr_session* s, const double* u, uint64_t u_len, double* r, char
   if (ok && !checked(s->arena->read_state(0, 2, r, s->stream), err, err_len, "AMR residual D2H")) return 1;
   saved.w_valid = 0;
   saved.r0_valid = 0;
-  saved.dt_min = 0x7ff0000000000000ull;
   if (!checked(s->arena->write_state(0, saved.cur, keep.data(), s->stream), err, err_len, "AMR state restore") ||
       !checked(copy_sync(s->arena->control(), &saved, sizeof(Control), hipMemcpyHostToDevice, s->stream), err, err_len,
                "AMR control restore"))
@@ -301,7 +299,6 @@ int amr_hip_monitor(amr_session* s, const double* region, const double* moment, 
   eval.active = 1;
   eval.bad = 0;
   eval.r0_valid = 0;
-  eval.dt_min = 0x7ff0000000000000ull;
   Control after{};
   std::vector<double> cells, walls;
   if (!checked(copy_sync(s->arena->control(), &eval, sizeof(Control), hipMemcpyHostToDevice, s->stream), err, err_len,
@@ -316,7 +313,6 @@ int amr_hip_monitor(amr_session* s, const double* region, const double* moment, 
     return 1;
   saved.w_valid = after.bad ? 0 : 1;
   saved.r0_valid = 0;
-  saved.dt_min = 0x7ff0000000000000ull;
   if (!checked(copy_sync(s->arena->control(), &saved, sizeof(Control), hipMemcpyHostToDevice, s->stream), err, err_len,
                "AMR control restore"))
     return 1;
@@ -341,7 +337,7 @@ int amr_hip_monitor(amr_session* s, const double* region, const double* moment, 
 int amr_hip_run(amr_session* s, double tend, int32_t trials, amr_state_meta* state, char* err, size_t err_len) {
   if (!s || !state || trials < 1 || !std::isfinite(tend) || tend < s->host_control->time)
     return fail(err, err_len, "invalid AMR GPU run");
-  hipamr::launch_target(s->arena->control(), 1, tend, INT64_MAX, nullptr, nullptr, s->stream);
+  hipamr::launch_target(s->arena->control(), s->arena->gather_lines(), 1, tend, INT64_MAX, nullptr, nullptr, s->stream);
   s->arena->launch_prims(s->stream);  // base primitives when the state was written by the host
   if (launch_trials(s, trials)) return fail(err, err_len, "AMR trial launch failed");
   if (!checked(hipGetLastError(), err, err_len, "AMR trial kernels") ||
@@ -359,7 +355,7 @@ int amr_hip_profile(amr_session* s, double tend, int32_t trials, amr_kernel_time
                     int32_t* count, char* err, size_t err_len) {
   if (!s || !out || !count || trials < 1 || capacity < 1 || !std::isfinite(tend) || tend < s->host_control->time)
     return fail(err, err_len, "invalid AMR GPU profile request");
-  hipamr::launch_target(s->arena->control(), 1, tend, INT64_MAX, nullptr, nullptr, s->stream);
+  hipamr::launch_target(s->arena->control(), s->arena->gather_lines(), 1, tend, INT64_MAX, nullptr, nullptr, s->stream);
   s->arena->launch_prims(s->stream);  // base primitives when the state was written by the host
   hipamr::EventHook hook(s->stream);
   for (int i = 0; i < trials; ++i) s->arena->launch_trial(s->stream, &hook);
@@ -523,7 +519,7 @@ extern "C" int amr_hip_run_noalloc(const amr_mesh_view* mesh, const amr_params* 
       hipamr::make_arena({in}, precision, tile, stream, &message, scratch_ptr[device], kScratchBytes);
   if (!arena) return fail(err, err_len, message);
   Control host{};
-  hipamr::launch_target(arena->control(), 1, tend, maxsteps, nullptr, nullptr, stream);
+  hipamr::launch_target(arena->control(), arena->gather_lines(), 1, tend, maxsteps, nullptr, nullptr, stream);
   arena->launch_prims(stream);
   bool expired = false;
   for (;;) {
