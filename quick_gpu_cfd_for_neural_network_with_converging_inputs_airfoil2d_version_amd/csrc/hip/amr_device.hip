@@ -86,11 +86,11 @@ inline int round_up(int n, int tile) { return (n + tile - 1) / tile * tile; }
 // blocks' latency, of which the rounds of face items are the largest part; beyond that the second
 // half of the kernel, which one thread per cell does, idles registers that other blocks need.
 // Trials of one mesh at 1 / 2 / 3 threads per cell: LF2 FP64 69 / 62 / 56 us, FP32 57 / 53 / 47;
-// level 7 FP64 77 / 70 / 64; level 8 FP64 (1640 tiles, over the line at 2) 124 / 128 / 132, FP32
-// 97 / 93 / 90.  8 LF2 meshes at tile 128, FP32, 73 / 67 / 64; 16 of mixed levels 103 / 101 / 117 and
-// FP64 176 / 210 / 273.
+// level 7 FP64 77 / 70 / 64; level 8 (1640 tiles) FP64, where two do not fit, 124 / 128 / 132, FP32
+// 97 / 93 / 90.  8 LF2 meshes at tile 128, FP32, 73 / 67 / 64, FP64 98 / 90; 16 of mixed levels FP32
+// 103 / 101 / 117 and FP64 176 / 210 / 273.
 int flux_spread_for(int tiles, int tile, int precision) {
-  const int resident = 256 * 4 * (precision == 64 ? 2 : 7);  // waves that the flux kernels' registers admit
+  const int resident = 256 * 4 * (precision == 64 ? 3 : 7);  // waves that the flux kernels' registers admit
   int spread = 3;
   while (spread > 1 && (tile * spread > 512 || static_cast<long long>(tiles) * (tile / 64) * spread > resident))
     --spread;

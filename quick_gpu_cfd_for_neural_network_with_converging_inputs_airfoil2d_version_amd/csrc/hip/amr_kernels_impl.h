@@ -593,12 +593,20 @@ __device__ __forceinline__ CellGrad<T> pick(bool first, const CellGrad<T>& a, co
                      first ? a.sx : b.sx, first ? a.sy : b.sy, first ? a.sdiff : b.sdiff};
 }
 
-// L, R (and Lg, Rg) are the records of the face's left and right cells; on a boundary face both
-// are the inside cell's.  `in`, `ing`: the evaluating cell, the inside cell of a boundary face.
+// Whether a face's gradient records are loaded after its inviscid flux instead of with its
+// primitives.  In FP64 that takes 26 registers off the stage passes (184 -> 158: three waves per SIMD
+// instead of two; 64 LF2 meshes 104 / 108 -> 88 / 91 us, 16 of mixed levels 173 -> 154 us a trial).  The
+// FP32 passes hold their waves either way and lose the loads' lead (136 / 141 -> 145 / 149 us on 256
+// LF2 meshes).
+template <class T>
+__device__ constexpr bool late_gradients() { return sizeof(T) == 8; }
+
+// L, R (and Lg, Rg, unless late_gradients) are the records of the face's left and right cells; on a
+// boundary face both are the inside cell's.  `in`: the inside cell of a boundary face.
 template <class T, bool BASE>
-__device__ __forceinline__ FaceFlux<T> face_flux(const MeshDesc<T>& d, int4 fi, const FaceGeo<T>& geo,
-                                                 const CellPrim<T>& in, const CellGrad<T>& ing, const CellPrim<T>& L,
-                                                 const CellPrim<T>& R, const CellGrad<T>& Lg, const CellGrad<T>& Rg) {
+__device__ __forceinline__ FaceFlux<T> face_flux(const ArenaPtrs<T>& a, const MeshDesc<T>& d, int4 fi,
+                                                 const FaceGeo<T>& geo, const CellPrim<T>& in, const CellPrim<T>& L,
+                                                 const CellPrim<T>& R, CellGrad<T> Lg, CellGrad<T> Rg) {
   FaceFlux<T> o{};
   o.ok = true;
   const int l = fi.x, r = fi.y, info = fi.z;
@@ -648,6 +656,11 @@ __device__ __forceinline__ FaceFlux<T> face_flux(const MeshDesc<T>& d, int4 fi, 
     // On an interior face every quantity taken from the inside cell below is replaced.
     const bool sa = d.sa != 0;
     const bool interior = side < 0;
+    if (late_gradients<T>()) {
+      Lg = load_grad(a, l >= 0 ? l : r);
+      Rg = load_grad(a, r >= 0 ? r : l);
+    }
+    const CellGrad<T>& ing = Lg;
     T g0 = ing.ux, g1 = ing.uy, g2 = ing.vx, g3 = ing.vy;
     const T rho_k = in.rho, u_k = in.u, v_k = in.v;
     const T eddy_k = sa ? in.eddy : T(0);
@@ -829,7 +842,8 @@ __device__ __forceinline__ void arrive_and_commit(Control* c, GatherLine* line, 
 // occupancy: base flux 151 -> 141 us with the batched entries below) and 7 in the stage passes
 // (72 VGPRs, 4 and 6 spilled; LDS for 14 blocks per CU).
 // On 256 LF2 meshes: base flux 187 -> 177 us, stage flux 188 -> 181 us against the unbounded
-// kernels; 8 waves (64 VGPRs) spills 11-14 and is slower.  FP64 (190-200 VGPRs) has no bound.
+// kernels; 8 waves (64 VGPRs) spills 11-14 and is slower.  FP64: 3 waves (157-167 VGPRs, no spill;
+// see late_gradients).
 // SPREAD threads per cell (1 to 3): a tile's face items are spread over SPREAD * tile threads,
 // the cell work stays on the first tile of them (a separate instantiation, so that the one-thread
 // kernel keeps its registers).  A tile touches 2.2 - 2.7 faces per cell, so three threads per cell
@@ -837,7 +851,7 @@ __device__ __forceinline__ void arrive_and_commit(Control* c, GatherLine* line, 
 // takes is its blocks' latency (see flux_spread_for).
 template <class T, int STAGE, int SPREAD>
 __global__ __launch_bounds__(SPREAD == 1 ? kMaxTile : kMaxThreads)
-__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (STAGE == 0 ? 5 : 7) : 1)))
+__attribute__((amdgpu_waves_per_eu(sizeof(T) == 4 ? (STAGE == 0 ? 5 : 7) : 3)))
 void k_flux(ArenaPtrs<T> a) {
   constexpr bool BASE = STAGE == 0;
   const int2 blk = cell_block(a);
@@ -889,9 +903,10 @@ void k_flux(ArenaPtrs<T> a) {
   bool ok = true;
   for (int c0 = range.x; c0 < range.y; c0 += chunk) {
     const int c1 = min(range.y, c0 + chunk);
-    // The base pass loads the next item's words while this one is evaluated (2 us less on 256
-    // LF2 meshes); the stage passes, held to 72 registers, would spill them and lose 9-11 us.
-    constexpr bool kPrefetch = BASE;
+    // The FP32 base pass loads the next item's words while this one is evaluated (2 us less on 256
+    // LF2 meshes); the stage passes, held to 72 registers, would spill them and lose 9-11 us, and the
+    // FP64 base pass keeps its third wave without them (101 -> 94 us on 64 LF2 meshes).
+    constexpr bool kPrefetch = BASE && sizeof(T) == 4;
     ItemWords<T> next{};
     if (kPrefetch && c0 + tid < c1) next = load_item_words(a.ITEM_A, static_cast<size_t>(c0 + tid));
     for (int i = c0 + tid; i < c1; i += nt) {
@@ -900,6 +915,7 @@ void k_flux(ArenaPtrs<T> a) {
       const FaceItem<T> it = item_of(words, a.ITEM_B, static_cast<size_t>(i));
       CellPrim<T> L{}, R{};
       CellGrad<T> Lg{}, Rg{};
+      const bool early = laminar && !late_gradients<T>();
       const int ll = it.left - first, rl = it.right - first;
       if (it.left >= 0) {
         if (ll >= 0 && ll < staged) {
@@ -907,7 +923,7 @@ void k_flux(ArenaPtrs<T> a) {
         } else {
           L = load_prim(a, rb, it.left);
         }
-        if (laminar) Lg = load_grad(a, it.left);
+        if (early) Lg = load_grad(a, it.left);
       }
       if (it.right >= 0) {
         if (rl >= 0 && rl < staged) {
@@ -915,7 +931,7 @@ void k_flux(ArenaPtrs<T> a) {
         } else {
           R = load_prim(a, rb, it.right);
         }
-        if (laminar) Rg = load_grad(a, it.right);
+        if (early) Rg = load_grad(a, it.right);
       }
       // A boundary face has one cell: it is the inside cell and both sides' record.
       if (it.left < 0) {
@@ -926,7 +942,7 @@ void k_flux(ArenaPtrs<T> a) {
         Rg = Lg;
       }
       const FaceFlux<T> f =
-          face_flux<T, BASE>(d, make_int4(it.left, it.right, it.info, 0), it.geo, L, Lg, L, R, Lg, Rg);
+          face_flux<T, BASE>(a, d, make_int4(it.left, it.right, it.info, 0), it.geo, L, L, R, Lg, Rg);
       ok = ok && f.ok;
       const int sl = i - c0;
       store4(slots.f + 4 * sl, f.f0, f.fx, f.fy, f.f3);
