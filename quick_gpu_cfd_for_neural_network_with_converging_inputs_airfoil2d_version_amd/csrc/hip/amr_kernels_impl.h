@@ -1006,28 +1006,53 @@ void k_flux(ArenaPtrs<T> a) {
     const T dt_area = BASE ? a.dt_area[k] : T(0);
     const T cell_vol = BASE && (laminar || sa) ? a.vol[k] : T(0);
     const T src_rate = BASE && sa ? a.SRATE[k] : T(0);
+    constexpr int kWalls = 2;
     if (w1 > w0) {
       const T snd = sqrt(d.gamma * p / rho);
-      for (int j = w0; j < w1; ++j) {
-        const T len = a.wall_len[j];
-        s1 += p * a.wall_nx[j] * len;
-        s2 += p * a.wall_ny[j] * len;
-        if (BASE) spectral += snd * len;
-        if (laminar) {
-          const int dn = a.wall_donor[j];
-          const int dl = dn - first;
-          const CellPrim<T> donor = dn == k ? own : (dl >= 0 && dl < staged ? tile_prim(lds, dl) : load_prim(a, rb, dn));
-          const T dd = a.wall_ddist[j];
-          T fv[4];
-          wall_shear(donor, a.wall_nx[j], a.wall_ny[j], dd, fv);
-          if (!isfinite(fv[1]) || !isfinite(fv[2])) ok = false;
-          s1 -= fv[1] * len;
-          s2 -= fv[2] * len;
-          if (BASE) diffusion += T(4.0 / 3.0) * fmax(donor.mu / donor.rho, own.mu / rho) / dd * len;
-          if (sa) {
-            const T coeff = donor.mu * T(1.0 / SaConst<T>::sigma) / dd * len;
-            sa_net -= -coeff * donor.phi;
-            if (BASE) sa_spec += coeff;
+      // The fragments kWalls at a time: their words together, then their donors' records (from the
+      // tile's LDS copy or the record arrays, by generic addresses), then the sums in their order.  A cell
+      // of an agglomerated mesh has up to eight fragments, and its block waited for two memory round
+      // trips after another for each, which a launch too small to hide them waits for.
+      for (int j0 = w0; j0 < w1; j0 += kWalls) {
+        T len[kWalls], nx[kWalls], ny[kWalls], dd[kWalls];
+        int dn[kWalls];
+#pragma unroll
+        for (int q = 0; q < kWalls; ++q) {
+          const int j = min(j0 + q, w1 - 1);  // fragments past the end are loaded in range and not summed
+          len[q] = a.wall_len[j];
+          nx[q] = a.wall_nx[j];
+          ny[q] = a.wall_ny[j];
+          dd[q] = laminar ? a.wall_ddist[j] : T(1);
+          dn[q] = laminar ? a.wall_donor[j] : k;
+        }
+        CellPrim<T> donor[kWalls];
+#pragma unroll
+        for (int q = 0; q < kWalls; ++q) {
+          const int dl = dn[q] - first;
+          const bool in_tile = dl >= 0 && dl < staged;
+          const T* const v = in_tile ? lds.v + 4 * dl : a.VREC[rb] + 4 * static_cast<size_t>(dn[q]);
+          const T* const w = in_tile ? lds.p + 4 * dl : a.PREC[rb] + prec_width<T>() * static_cast<size_t>(dn[q]);
+          load4(v, donor[q].rho, donor[q].u, donor[q].v, donor[q].phi);
+          donor[q].mu = w[1];
+        }
+#pragma unroll
+        for (int q = 0; q < kWalls; ++q) {
+          if (j0 + q >= w1) break;
+          s1 += p * nx[q] * len[q];
+          s2 += p * ny[q] * len[q];
+          if (BASE) spectral += snd * len[q];
+          if (laminar) {
+            T fv[4];
+            wall_shear(donor[q], nx[q], ny[q], dd[q], fv);
+            if (!isfinite(fv[1]) || !isfinite(fv[2])) ok = false;
+            s1 -= fv[1] * len[q];
+            s2 -= fv[2] * len[q];
+            if (BASE) diffusion += T(4.0 / 3.0) * fmax(donor[q].mu / donor[q].rho, own.mu / rho) / dd[q] * len[q];
+            if (sa) {
+              const T coeff = donor[q].mu * T(1.0 / SaConst<T>::sigma) / dd[q] * len[q];
+              sa_net -= -coeff * donor[q].phi;
+              if (BASE) sa_spec += coeff;
+            }
           }
         }
       }
