@@ -72,7 +72,11 @@ constexpr int kItemInfoMask = 15;
 // 5/2, 11/4 and 3 per cell give 164, 164, 178, 159, 171 and 171 us for the base pass and 700,
 // 699, 705, 683, 690 and 691 us per batch step (one chunk round for most tiles against losing a
 // block per CU); a stage chunk of 11/4 gains nothing, 3 loses 13 us per stage pass.
-__host__ __device__ constexpr int item_chunk(int tile, bool) { return tile * 5 / 2; }
+__host__ __device__ constexpr int item_round(int tile) { return tile * 5 / 2; }
+// With three threads per cell a chunk is two rounds: such launches leave LDS to spare, and a tile of more
+// than 5/2 items per cell (in one of ten tiles of an LF2 mesh) evaluated the rest after a barrier, 3 us
+// of a launch's 11.  A cell sums its faces round by round whatever the chunk, so the bits stay.
+__host__ __device__ constexpr int item_chunk(int tile, int spread) { return (spread == 3 ? 2 : 1) * item_round(tile); }
 
 // One LSQ gradient term of a cell: its source (>= 0 cell, -1 body wall, -2 - side: no-slip domain
 // side) and its two weights, fetched by one load (12 bytes in FP32) instead of three.
@@ -94,8 +98,8 @@ struct TermRec<double> {
 // flux) in the base pass.
 // Gradient launches: 4 T per cell.
 template <class T>
-constexpr size_t flux_lds_bytes(int tile, bool base) {
-  return (static_cast<size_t>(tile) * 8 + static_cast<size_t>(item_chunk(tile, base)) * (base ? 8 : 5)) * sizeof(T);
+constexpr size_t flux_lds_bytes(int tile, bool base, int spread) {
+  return (static_cast<size_t>(tile) * 8 + static_cast<size_t>(item_chunk(tile, spread)) * (base ? 8 : 5)) * sizeof(T);
 }
 template <class T>
 constexpr size_t grad_lds_bytes(int tile) {

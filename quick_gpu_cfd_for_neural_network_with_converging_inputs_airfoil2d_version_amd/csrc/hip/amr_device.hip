@@ -788,7 +788,8 @@ class DeviceArena final : public Arena {
     if (hipGetDevice(&device) != hipSuccess ||
         hipDeviceGetAttribute(&lds_max, hipDeviceAttributeMaxSharedMemoryPerBlock, device) != hipSuccess)
       return "AMR device query failed";
-    if (flux_lds_bytes<T>(tile_, true) > static_cast<size_t>(lds_max))
+    if (flux_lds_bytes<T>(tile_, true, flux_spread_for(n_cell_blocks_, tile_, sizeof(T) == 8 ? 64 : 32)) >
+        static_cast<size_t>(lds_max))
       return "AMR tile needs more LDS per block than the device provides";
     if (external_) {
       if (slab_bytes_ > external_bytes_)

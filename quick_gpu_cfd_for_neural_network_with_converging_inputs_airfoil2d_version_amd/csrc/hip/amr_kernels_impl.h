@@ -200,8 +200,7 @@ struct FaceSlots {
   T* f;
   T* sf;  // stage passes
   T* x;   // base pass
-  __device__ FaceSlots(int tile, bool base)
-      : f(reinterpret_cast<T*>(tile_lds) + 8 * tile), sf(f + 4 * item_chunk(tile, base)), x(sf) {}
+  __device__ FaceSlots(int tile, int chunk) : f(reinterpret_cast<T*>(tile_lds) + 8 * tile), sf(f + 4 * chunk), x(sf) {}
 };
 
 template <class T>
@@ -878,7 +877,8 @@ void k_flux(ArenaPtrs<T> a) {
   const int bit = BASE ? BAD_BASE : BAD_STAGE;
   const int staged = min(tn, d.cell_begin + d.n_cells - first);  // valid cells of the tile
   const TileCells<T> lds(tn);
-  const FaceSlots<T> slots(tn, BASE);
+  const int chunk = item_chunk(tn, SPREAD);
+  const FaceSlots<T> slots(tn, chunk);
   __shared__ int failed;  // block snapshot of the slot's admissibility bits (or the trial ended)
   if (tid == 0) failed = live ? c->bad : 1;
   // The cell's face-entry range is loaded with its record instead of after the barrier (stage
@@ -898,7 +898,6 @@ void k_flux(ArenaPtrs<T> a) {
   // order.  A face shared with another tile is evaluated by both tiles from the same inputs, so
   // both cells see the same bits.
   const int2 range = a.item_range[tile];
-  const int chunk = item_chunk(tn, BASE);
   T s0 = 0, s1 = 0, s2 = 0, s3 = 0, spectral = 0, diffusion = 0, sa_net = 0, sa_spec = 0;
   bool ok = true;
   for (int c0 = range.x; c0 < range.y; c0 += chunk) {
@@ -956,7 +955,10 @@ void k_flux(ArenaPtrs<T> a) {
       // so the cell waits for one memory round trip per batch instead of one per face (stage flux
       // 157 / 167 -> 155 / 160 us on 256 LF2 meshes; base flux 151 -> 141 us once its register
       // bound no longer made it spill).
-      const int lo = c0 - range.x, n_slots = c1 - c0;
+      // Rounds of the chunk's slots: one, or two with three threads per cell.
+      const int round = item_round(tn);
+      for (int r0 = c0; r0 < c1; r0 += round) {
+      const int lo = c0 - range.x, from = r0 - c0, n_slots = min(c1, r0 + round) - c0;
       const int begin = csr_begin, end = csr_end;
       constexpr int kEntries = 4;
       for (int j0 = begin; j0 < end; j0 += kEntries) {
@@ -967,7 +969,7 @@ void k_flux(ArenaPtrs<T> a) {
         for (int q = 0; q < kEntries; ++q) {
         const int e = ent[q];
         const int sl = (e >> 1) - lo;
-        if (j0 + q >= end || sl < 0 || sl >= n_slots) continue;
+        if (j0 + q >= end || sl < from || sl >= n_slots) continue;
         const T sgn = (e & 1) ? T(-1) : T(1);
         T f0, fx, fy, f3;
         load4(slots.f + 4 * sl, f0, fx, fy, f3);
@@ -986,6 +988,8 @@ void k_flux(ArenaPtrs<T> a) {
           sa_net += sgn * slots.sf[sl];
         }
         }
+      }
+      if (SPREAD != 3) break;
       }
     }
     __syncthreads();  // the next chunk reuses the slots
@@ -1011,8 +1015,8 @@ void k_flux(ArenaPtrs<T> a) {
       const T snd = sqrt(d.gamma * p / rho);
       // The fragments kWalls at a time: their words together, then their donors' records (from the
       // tile's LDS copy or the record arrays, by generic addresses), then the sums in their order.  A cell
-      // of an agglomerated mesh has up to eight fragments, and its block waited for two memory round
-      // trips after another for each, which a launch too small to hide them waits for.
+      // of an agglomerated mesh has up to eight fragments, each two memory round trips after another
+      // (batch step of 256 LF2 meshes 594 -> 585 us, 587 with four; 64 in FP64 345 -> 341).
       for (int j0 = w0; j0 < w1; j0 += kWalls) {
         T len[kWalls], nx[kWalls], ny[kWalls], dd[kWalls];
         int dn[kWalls];
@@ -1441,7 +1445,7 @@ inline int blocks_of(int n, int tile) { return (n + tile - 1) / tile; }
 template <class T>
 int launch_base_pass(const ArenaPtrs<T>& a, hipStream_t s, LaunchHook* hook) {
   const dim3 tile(a.tile), cells(a.n_grid_blocks);
-  const size_t base_lds = flux_lds_bytes<T>(a.tile, true), vel_lds = grad_lds_bytes<T>(a.tile);
+  const size_t base_lds = flux_lds_bytes<T>(a.tile, true, a.flux_spread), vel_lds = grad_lds_bytes<T>(a.tile);
   int launches = 0;
   if (a.any_laminar) HIPAMR_LAUNCH_LDS("gradient_base", (k_grad<T, 0>), cells, vel_lds, a);
   HIPAMR_LAUNCH_FLUX("flux_base", 0, cells, base_lds, a);
@@ -1470,7 +1474,7 @@ int launch_residual(const ArenaPtrs<T>& a, hipStream_t s, LaunchHook* hook) {
 template <class T>
 int launch_trial(const ArenaPtrs<T>& a, hipStream_t s, LaunchHook* hook) {
   const dim3 tile(a.tile), cells(a.n_grid_blocks);
-  const size_t stage_lds = flux_lds_bytes<T>(a.tile, false), vel_lds = grad_lds_bytes<T>(a.tile);
+  const size_t stage_lds = flux_lds_bytes<T>(a.tile, false, a.flux_spread), vel_lds = grad_lds_bytes<T>(a.tile);
   int launches = launch_base_pass(a, s, hook);
   HIPAMR_LAUNCH("stage0", k_stage0<T>, cells, a);
   if (a.any_small) {
