@@ -178,8 +178,8 @@ class Batch:
         return _states(self._state_buf)
 
     def download(self, slot: int) -> tuple[np.ndarray, dict]:
-        n_cells = self.states()[slot]["n_cells"]
-        u = np.zeros(self.nv * n_cells)
+        self._lib.amr_batch_slots(self.handle, self._state_buf)
+        u = np.empty(self.nv * self._state_buf[slot].n_cells)
         meta = N.amr_state_meta()
         err = N.err_buffer()
         self._check(self._lib.amr_batch_download(self.handle, slot, N.dptr(u), u.size, C.byref(meta), err,

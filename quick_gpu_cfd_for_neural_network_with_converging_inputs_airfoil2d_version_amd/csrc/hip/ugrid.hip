@@ -1310,6 +1310,42 @@ __global__ __launch_bounds__(kThreads) void k_srd_apply(Grid g) {
   if (__any(bad) && lane == 0) atomicOr(&c->bad, 1);
 }
 
+// The two ghost layers of every plane of `out` from the interior of `in` (fill_ghosts on the device,
+// for axes of at least two cells, where every ghost maps to an interior cell).  One block per plane
+// and row: a row beside the interior has 2 kGhosts ghosts, a row above or below it is all ghosts.
+__global__ __launch_bounds__(kThreads) void k_fill_ghosts(Grid g, const double* in, double* out) {
+  const int jj = blockIdx.x, j = jj - kGhosts;
+  const size_t plane = static_cast<size_t>(blockIdx.y) * g.plane;
+  const int v = blockIdx.y % 4;
+  const auto mapped = [](int k, int n, int lo, int hi, bool* flip) {
+    if (k < 0) {
+      if (lo == BC_PERIODIC) return k + n;
+      *flip = lo == BC_REFLECT;
+      return lo == BC_REFLECT ? -k - 1 : 0;
+    }
+    if (k >= n) {
+      if (hi == BC_PERIODIC) return k - n;
+      *flip = hi == BC_REFLECT;
+      return hi == BC_REFLECT ? 2 * n - 1 - k : n - 1;
+    }
+    return k;
+  };
+  bool flip_v = false;
+  const int js = mapped(j, g.ny, g.bc[2], g.bc[3], &flip_v);
+  const bool inside = j >= 0 && j < g.ny;
+  const int count = inside ? 2 * kGhosts : g.mx;
+  for (int q = threadIdx.x; q < count; q += blockDim.x) {
+    const int ii = inside && q >= kGhosts ? g.nx + q : q;
+    bool flip_u = false;
+    const int is = mapped(ii - kGhosts, g.nx, g.bc[0], g.bc[1], &flip_u);
+    double sign = 1.0;
+    if (v == 1 && flip_u) sign = -sign;
+    if (v == 2 && flip_v) sign = -sign;
+    out[plane + static_cast<size_t>(jj) * g.mx + ii] =
+        sign * in[plane + static_cast<size_t>(js + kGhosts) * g.mx + is + kGhosts];
+  }
+}
+
 __global__ void k_zero(double* p, size_t n) {
   for (size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; q < n;
        q += static_cast<size_t>(gridDim.x) * blockDim.x)
@@ -1336,8 +1372,6 @@ struct ugrid_session {
   hipStream_t stream = nullptr;
   hipGraphExec_t exec = nullptr;
   int graph_trials = 0;
-  std::vector<double> uploaded;  // the state as uploaded (its ghost cells are the download's
-                                 // ghosts until a step begins)
   std::vector<void*> owned;
 };
 
@@ -1784,7 +1818,7 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   const hipMemcpyKind h2d = hipMemcpyHostToDevice;
   const size_t bytes = states * sizeof(double);
   // Every buffer that can come to hold the accepted state starts as the upload, so its ghost
-  // cells are the entry values (the device never writes ghost cells).
+  // cells are the entry values (only a download after the first step writes ghost cells).
   if (!ok(hipMemcpyAsync(g.B[0], u, bytes, h2d, s->stream), err, err_len, "upload state") ||
       !ok(hipMemcpyAsync(g.B[1], u, bytes, h2d, s->stream), err, err_len, "upload state") ||
       !ok(hipMemcpyAsync(g.B[2], u, bytes, h2d, s->stream), err, err_len, "upload state") ||
@@ -1808,7 +1842,6 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
     release(s);
     return 3;
   }
-  s->uploaded.assign(u, u + states);
   s->mco = mco;
   if (setup->cut && !upload_cut(s, *setup->cut, setup->dx, setup->dy, err, err_len)) {
     release(s);
@@ -1905,15 +1938,26 @@ extern "C" int ugrid_download(ugrid_session* s, double* u, uint64_t u_len, doubl
       !ok(hipStreamSynchronize(s->stream), err, err_len, "control"))
     return 3;
   const size_t bytes = s->states * sizeof(double);
-  if (u) {
+  // Once a step has begun, the ghosts are a boundary fill that the device makes in the accepted
+  // state's own buffer (its kernels never read ghost cells): one copy, instead of a second state
+  // beside it and two passes of the host over both (8 cases of 1024 x 1024: 123 -> 15 ms with the
+  // mirror's pull in place).
+  if (u && c.ghost_from != 0 && g.nx >= 2 && g.ny >= 2 && g.my <= 65535 && 4LL * g.ncase <= 65535) {
+    const double* from = c.ghost_from == 1 ? g.B[c.cur] : g.B[c.cur ^ 1];
+    hipLaunchKernelGGL(k_fill_ghosts, dim3(g.my, 4 * g.ncase), dim3(kThreads), 0, s->stream, g, from, g.B[c.cur]);
+    if (!ok(hipGetLastError(), err, err_len, "ghost cells") ||
+        !ok(hipMemcpyAsync(u, g.B[c.cur], bytes, hipMemcpyDeviceToHost, s->stream), err, err_len, "download") ||
+        !ok(hipStreamSynchronize(s->stream), err, err_len, "download"))
+      return 3;
+  } else if (u) {
     if (!ok(hipMemcpyAsync(u, g.B[c.cur], bytes, hipMemcpyDeviceToHost, s->stream), err, err_len, "download") ||
         !ok(hipStreamSynchronize(s->stream), err, err_len, "download"))
       return 3;
+    // (Before the first step, and in backward Euler, every buffer's ghosts are still the uploaded ones.)
     std::vector<double> other;
-    const double* ghosts = s->uploaded.data();
+    const double* ghosts = nullptr;
     if (c.ghost_from == 1) {
       fill_ghosts(g, u);
-      ghosts = nullptr;
     } else if (c.ghost_from == 2) {
       other.resize(s->states);
       if (!ok(hipMemcpyAsync(other.data(), g.B[c.cur ^ 1], bytes, hipMemcpyDeviceToHost, s->stream), err, err_len,

@@ -291,12 +291,15 @@ class DeviceSession:
     def pull(self) -> None:
         s = self.solver
         err = N.err_buffer()
-        u = np.empty_like(s.U)
+        # Straight into the solver's own array where its layout allows (a state is hundreds of megabytes).
+        own = s.U.dtype == np.float64 and s.U.flags.c_contiguous and s.U.flags.writeable
+        u = s.U if own else np.empty(s.U.shape)
         t = np.empty(s.ncase)
         dt = np.empty(s.ncase)
         if self.lib.ugrid_download(self.handle, N.dptr(u), u.size, N.dptr(t), N.dptr(dt), err, N.ERR_LEN):
             raise RuntimeError(err.value.decode())
-        s.U[:] = u
+        if not own:
+            s.U[:] = u
         s.t[:] = t
         s.dt[:] = dt
         s.nsteps += self.meta.nsteps - self._counted[0]
