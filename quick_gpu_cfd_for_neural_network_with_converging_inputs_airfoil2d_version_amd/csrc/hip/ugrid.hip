@@ -60,7 +60,7 @@ enum : int { BC_PERIODIC = 0, BC_TRANSMISSIVE = 1, BC_REFLECT = 2 };
 enum : int { RUNNING = -1 };
 // Backward-Euler phases of a physical step (each kernel of the replayed sequence acts only in its
 // phase; the one-wave decision kernels move the phase).
-enum : int { PH_BOUND = 0, PH_COPY = 1, PH_RES = 2, PH_TRIAL = 3 };
+enum : int { PH_BOUND = 0, PH_COPY = 1, PH_UPDATE = 2, PH_RETRY = 3 };
 // Why a backward-Euler run stopped with 2, 3 or 4.
 enum : int { WHY_NONE = 0, WHY_INITIAL = 1, WHY_PSEUDO = 2, WHY_DEFECT = 3, WHY_MAXITER = 4, WHY_DT = 5 };
 
@@ -102,7 +102,6 @@ struct Grid {
   // State buffers: B[0] and B[1] alternate as accepted state and RK candidate, B[2] holds the
   // second RK stage; backward Euler rotates all three (accepted state, iterate, candidate).
   double* B[3];
-  double* R;           // residual of the backward-Euler iterate
   double* t;
   double* dt;          // step of the running trial
   double* dt_out;      // last accepted step
@@ -535,8 +534,14 @@ __device__ void commit(const Grid& g, unsigned long long* s_max) {
 //   MODE 2: S2 = 3/4 U + 1/4 (U1 + dt L(U1))          (U1 in U[cur^1])
 //   MODE 3: U[cur^1] = 1/3 U + 2/3 (S2 + dt L(S2)), and the candidate's wave-speed bound
 //   MODE 0: R = L(in)
-//   MODE 4: R = L(Q), per case max over cells of max_v |dt R - (Q - U)| / max(1, |U|)
-//           (infinite for a non-finite defect), src/euler2d_cuda.cu:331-350
+//   MODE 4: one pseudo update of backward Euler: per case the maximum over cells of the scaled defect
+//           max_v |D| / max(1, |U|), D = dt L(Q) - (Q - U) (infinite for a non-finite defect;
+//           src/euler2d_cuda.cu:331-350), and the candidate Q + omega D, omega = cfl* / (cfl* + dt
+//           rate(Q)), of the cases that move, with its admissibility.  The candidate is formed before
+//           k_be_decide has judged the defect and is dropped when that ends the step, so that an update
+//           is two launches and reads the states once: on 8 cases of 256 x 256 59 -> 33 us against a
+//           residual, a decision, a candidate and a check kernel.  A candidate that is refused is formed
+//           again, with its residual, at half the pseudo CFL.
 // ---------------------------------------------------------------------------------------------
 __device__ __forceinline__ void load_row(const double* p, size_t plane, double (&c)[4]) {
   for (int v = 0; v < 4; ++v) c[v] = p[v * plane];
@@ -557,8 +562,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
   if (MODE > 0) {
     if (__hip_atomic_load(&ctrl->status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != RUNNING) return;
     if (MODE == 4) {
-      const int phase = ctrl->phase;
-      if (phase != PH_COPY && phase != PH_RES) return;
+      if (ctrl->phase == PH_BOUND) return;
       qb = ctrl->qbuf;
     } else {
       skip = __hip_atomic_load(&ctrl->bad, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
@@ -568,7 +572,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
   const double* base = MODE > 0 ? g.B[cur] : nullptr;
   const double* in = MODE == 0 ? rhs_in : MODE == 1 ? g.B[cur] : MODE == 2 ? g.B[cur ^ 1] : MODE == 3 ? g.B[2]
                                                                                                     : g.B[qb];
-  double* out = MODE == 0 ? rhs_out : MODE == 2 ? g.B[2] : MODE == 4 ? g.R : g.B[cur ^ 1];
+  double* out = MODE == 0 ? rhs_out : MODE == 2 ? g.B[2] : MODE == 4 ? g.B[3 - cur - qb] : g.B[cur ^ 1];
+  const double pseudo = MODE == 4 ? ctrl->pseudo : 0.0;
   constexpr double A = MODE == 2 ? 0.75 : MODE == 3 ? 1.0 / 3.0 : 0.0;
   constexpr double B = MODE == 2 ? 0.25 : MODE == 3 ? 2.0 / 3.0 : 1.0;
 
@@ -601,6 +606,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
     unsigned plain = 0u;
     Flux gprev{}, xres{};  // xres: x residual of a full cell, or ae FX_e - aw FX_w of a cut cell
     double ay_prev = 1.0;  // aperture of the previous y face (cut grids)
+    double ax_sum = 0.0;   // cut grids, MODE 4: apertures of the previous row's x faces
     double q0 = 0, q1 = 0, q2 = 0, q3 = 0;  // conserved state of the owned cell of the previous row
     unsigned code_prev = 0;                  // cut grids: code of the lane's cell of the previous row
     const bool in_x = i >= 0 && i <= g.nx;   // the lane's west x face is a grid face
@@ -618,8 +624,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
         load_row(in + case_base + static_cast<size_t>(jc + kGhosts) * g.mx, plane, next);
       }
       double base_row[4];
-      if (MODE > 1 && MODE < 4 && j > j0 && owner)
-        for (int v = 0; v < 4; ++v) base_row[v] = __builtin_nontemporal_load(base + ko + v * plane);
+      if (MODE > 1 && j > j0 && owner)
+        for (int v = 0; v < 4; ++v) base_row[v] = MODE == 4 ? base[ko + v * plane] : __builtin_nontemporal_load(base + ko + v * plane);
       // Cut grids: codes of the mapped cell (solid or not) and of the lane's own column at row j
       // (its faces, cut or not, rewritten by SRD or not).
       const unsigned code_m = CUT ? g.code[static_cast<size_t>(jm + kGhosts) * g.mx + ic + kGhosts] : 0u;
@@ -684,25 +690,45 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
             r2 -= iv * pw * g.way[kc];
           }
           if (CUT && MODE == 3) moved = (code_prev & 4u) != 0u;
-          if (MODE == 0 || MODE == 4) {
+          if (MODE == 0) {
             out[ko] = r0;
             out[ko + plane] = r1;
             out[ko + 2 * plane] = r2;
             out[ko + 3 * plane] = r3;
-            if (MODE == 4 && dt > 0.0 && fluid) {
+          } else if (MODE == 4) {
+            if (dt > 0.0 && fluid) {
               const double r[4] = {r0, r1, r2, r3}, q[4] = {q0, q1, q2, q3};
-              double norm = 0.0;
+              double defect[4], norm = 0.0;
+              bool finite = true;
               for (int v = 0; v < 4; ++v) {
-                const double old = base[ko + v * plane];
-                const double defect = dt * r[v] - (q[v] - old);
-                if (!isfinite(defect)) {
-                  norm = HUGE_VAL;
-                  break;
-                }
-                norm = fmax(norm, fabs(defect) / fmax(1.0, fabs(old)));
+                const double old = base_row[v];
+                defect[v] = dt * r[v] - (q[v] - old);
+                finite = finite && isfinite(defect[v]);
+                norm = fmax(norm, fabs(defect[v]) / fmax(1.0, fabs(old)));
               }
+              if (!finite) norm = HUGE_VAL;
               const unsigned long long bits = static_cast<unsigned long long>(__double_as_longlong(norm));
               bound = bits > bound ? bits : bound;
+              double rate;
+              if (CUT) {
+                // implicit_spectral_rate of a cell of a cut grid (src/implicit2d.h:33-43)
+                const double wx = g.wax[kc], wy = g.way[kc];
+                const double wall = sqrt(wx * wx + wy * wy);
+                rate = ((fabs(wprev.u) + wprev.a) * ax_sum + (fabs(wprev.v) + wprev.a) * (ay + ay_prev) +
+                        fabs(wprev.u * wx + wprev.v * wy) + wprev.a * wall) /
+                       (2.0 * g.vol[kc]);
+              } else if (plain & 2u) {
+                rate = quot<true>(fabs(wprev.u) + wprev.a, dxi, rdxi) + quot<true>(fabs(wprev.v) + wprev.a, dyj, rdyj);
+              } else {
+                rate = (fabs(wprev.u) + wprev.a) / dxi + (fabs(wprev.v) + wprev.a) / dyj;
+              }
+              const double omega = pseudo / (pseudo + dt * rate);
+              double n[4];
+              for (int v = 0; v < 4; ++v) {
+                n[v] = q[v] + omega * defect[v];
+                out[ko + v * plane] = n[v];
+              }
+              if (check_candidate<false>(n[0], n[1], n[2], n[3], g, dxi, dyj, rdxi, rdyj, nullptr)) wave_bad = true;
             }
           } else {
             double a0 = q0, a1 = q1, a2 = q2, a3 = q3;
@@ -757,6 +783,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
                          : face_flux<true, AUSM, false>(g.gamma, mco, wl, w);
         const Flux fe{shfl_down1(fw.m), shfl_down1(fw.x), shfl_down1(fw.y), shfl_down1(fw.e)};
         const double ae = CUT ? shfl_down1(ax) : 1.0;
+        if (CUT && MODE == 4) ax_sum = ae + ax;
         if (CUT && owner && (code_u & 2u))
           xres = Flux{ae * fe.m - ax * fw.m, ae * fe.x - ax * fw.x, ae * fe.y - ax * fw.y, ae * fe.e - ax * fw.e};
         else if (plain_row)
@@ -772,6 +799,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
   }
   if (MODE == 0) return;
   if (MODE == 4) {
+    if (__any(wave_bad) && lane == 0) atomicOr(&ctrl->bad, 1);
     bound = wave_max(bound);
     if (work && lane == 0) {
       if (g.use_part)
@@ -875,9 +903,10 @@ __global__ __launch_bounds__(kThreads) void k_open(Grid g, double tend, long lon
 }
 
 // ------------------------------------------------------------------ backward Euler --
-// src/euler2d_cuda.cu:370-447 with src/implicit2d.h:16-63 and src/implicit2d.cpp:37-69.  A replay
-// runs k_bound, k_be_open, k_be_copy, k_stage<4>, k_be_decide, k_be_trial, k_be_check; each acts
-// only in its phase, so one replay completes at least one phase.
+// src/euler2d_cuda.cu:370-447 with src/implicit2d.h:16-63 and src/implicit2d.cpp:37-69.  A round is
+// k_bound, k_be_open, k_be_copy, which open a physical step, and kUpdates pairs of k_stage<4> and
+// k_be_decide, each a pseudo update; every kernel acts only in its phase, so a round completes at
+// least one phase.
 
 // Nonphysical interior cells of B[cur] (the run's initial check).  Grid-stride over all cases.
 __global__ __launch_bounds__(kThreads) void k_check_state(Grid g) {
@@ -1004,137 +1033,97 @@ __global__ __launch_bounds__(kThreads) void k_be_copy(Grid g) {
   }
 }
 
-// Convergence of the pseudo iteration (implicit2d_converged): tolerance max(atol, rtol * the
-// step's first norm) per case; on convergence the iterate becomes the accepted state and the
-// clocks advance (implicit2d_advance_time), else a candidate follows or the iteration limit
-// ends the run with 4.
+// The decision on a pseudo update.  Convergence of the iteration (implicit2d_converged): tolerance
+// max(atol, rtol * the step's first norm) per case; on convergence the iterate becomes the accepted
+// state and the clocks advance (implicit2d_advance_time), at the iteration limit the run ends with 4.
+// Else the candidate becomes the next iterate, or, inadmissible, the pseudo CFL is halved for another
+// (12 retries, then 2); a retry judges its candidate only.
 __global__ __launch_bounds__(kDecide) void k_be_decide(Grid g) {
   __shared__ unsigned long long s_max[kPartCases];
   Control* c = g.ctrl;
-  if (c->status != RUNNING || (c->phase != PH_COPY && c->phase != PH_RES)) return;
-  __syncthreads();  // every wave has read the phase that the first one moves
-  if (g.use_part) reduce_parts(g, s_max);
+  const int phase = c->phase;
+  if (c->status != RUNNING || phase == PH_BOUND) return;
+  const bool bad = c->bad != 0;
+  __syncthreads();  // every wave has read the phase and the flag that the first one moves
+  const bool retry = phase == PH_RETRY;
+  if (g.use_part && !retry) reduce_parts(g, s_max);
   if (threadIdx.x >= kLanes) return;
   const unsigned long long* norms = g.use_part ? s_max : g.norm;
   const int lane = threadIdx.x;
-  int nonfinite = 0;
-  for (int k = lane; k < g.ncase; k += kLanes)
-    if (!isfinite(__longlong_as_double(static_cast<long long>(norms[k])))) nonfinite = 1;
-  if (__any(nonfinite)) {
-    for (int k = lane; k < g.ncase; k += kLanes) g.norm[k] = 0;
-    if (lane == 0) {
-      c->status = 2;
-      c->reason = WHY_DEFECT;
-      c->events += 1;
+  if (!retry) {
+    int nonfinite = 0;
+    for (int k = lane; k < g.ncase; k += kLanes)
+      if (!isfinite(__longlong_as_double(static_cast<long long>(norms[k])))) nonfinite = 1;
+    if (__any(nonfinite)) {
+      for (int k = lane; k < g.ncase; k += kLanes) g.norm[k] = 0;
+      if (lane == 0) {
+        c->status = 2;
+        c->reason = WHY_DEFECT;
+        c->bad = 0;
+        c->events += 1;
+      }
+      return;
     }
-    return;
-  }
-  const bool first = c->iter == 0;
-  unsigned long long imax = 0, nmax = 0, tmax = 0;
-  int open = 0;
-  for (int k = lane; k < g.ncase; k += kLanes) {
-    const double norm = __longlong_as_double(static_cast<long long>(norms[k]));
-    if (first) g.initial[k] = norm;
-    const double initial = g.initial[k];
-    const double tol = fmax(g.atol, g.rtol * initial);
-    const unsigned long long bi = static_cast<unsigned long long>(__double_as_longlong(initial));
-    const unsigned long long bn = static_cast<unsigned long long>(__double_as_longlong(norm));
-    const unsigned long long bt = static_cast<unsigned long long>(__double_as_longlong(tol));
-    imax = bi > imax ? bi : imax;
-    nmax = bn > nmax ? bn : nmax;
-    tmax = bt > tmax ? bt : tmax;
-    if (!isfinite(tol) || norm > tol) open = 1;
-    g.norm[k] = 0;
-  }
-  imax = wave_max(imax);
-  nmax = wave_max(nmax);
-  tmax = wave_max(tmax);
-  const bool converged = !__any(open);
-  if (converged) {
-    const double tend = c->tend;
+    const bool first = c->iter == 0;
+    unsigned long long imax = 0, nmax = 0, tmax = 0;
+    int open = 0;
     for (int k = lane; k < g.ncase; k += kLanes) {
-      const double d = g.dt[k];
-      if (d <= 0.0) continue;
-      const double t = g.t[k];
-      g.t[k] = d == tend - t ? tend : t + d;
+      const double norm = __longlong_as_double(static_cast<long long>(norms[k]));
+      if (first) g.initial[k] = norm;
+      const double initial = g.initial[k];
+      const double tol = fmax(g.atol, g.rtol * initial);
+      const unsigned long long bi = static_cast<unsigned long long>(__double_as_longlong(initial));
+      const unsigned long long bn = static_cast<unsigned long long>(__double_as_longlong(norm));
+      const unsigned long long bt = static_cast<unsigned long long>(__double_as_longlong(tol));
+      imax = bi > imax ? bi : imax;
+      nmax = bn > nmax ? bn : nmax;
+      tmax = bt > tmax ? bt : tmax;
+      if (!isfinite(tol) || norm > tol) open = 1;
+      g.norm[k] = 0;
     }
-  }
-  if (lane == 0) {
-    c->initial_defect = __longlong_as_double(static_cast<long long>(imax));
-    c->final_defect = __longlong_as_double(static_cast<long long>(nmax));
-    c->tolerance = __longlong_as_double(static_cast<long long>(tmax));
-    c->checks += 1;
+    imax = wave_max(imax);
+    nmax = wave_max(nmax);
+    tmax = wave_max(tmax);
+    const bool converged = !__any(open);
     if (converged) {
-      c->cur = c->qbuf;
-      c->nsteps += 1;
-      c->steps += 1;
-      c->phase = PH_BOUND;
-    } else if (c->iter >= g.maxiter) {
-      c->status = 4;
-      c->reason = WHY_MAXITER;
-    } else {
-      c->phase = PH_TRIAL;
+      const double tend = c->tend;
+      for (int k = lane; k < g.ncase; k += kLanes) {
+        const double d = g.dt[k];
+        if (d <= 0.0) continue;
+        const double t = g.t[k];
+        g.t[k] = d == tend - t ? tend : t + d;
+      }
+    }
+    const bool limit = !converged && c->iter >= g.maxiter;
+    if (lane == 0) {
+      c->initial_defect = __longlong_as_double(static_cast<long long>(imax));
+      c->final_defect = __longlong_as_double(static_cast<long long>(nmax));
+      c->tolerance = __longlong_as_double(static_cast<long long>(tmax));
+      c->checks += 1;
       c->pretries = 0;
-    }
-    c->events += 1;
-  }
-}
-
-// Pseudo-time candidate: trial = Q + omega (dt R - (Q - U)), omega = cfl* / (cfl* + dt rate(Q))
-// for the cases that move, then the admissibility of every case's candidate cells.
-__global__ __launch_bounds__(kThreads) void k_be_trial(Grid g) {
-  const Control* c = g.ctrl;
-  if (c->status != RUNNING || c->phase != PH_TRIAL) return;
-  const int cur = c->cur, qb = c->qbuf, tb = 3 - cur - qb;
-  const double pseudo = c->pseudo;
-  const double* u = g.B[cur];
-  const double* Q = g.B[qb];
-  double* trial = g.B[tb];
-  const size_t inner = static_cast<size_t>(g.nx) * g.ny;
-  const size_t pl = g.plane;
-  bool bad = false;
-  for (size_t q = blockIdx.x * static_cast<size_t>(blockDim.x) + threadIdx.x; q < inner * g.ncase;
-       q += static_cast<size_t>(gridDim.x) * blockDim.x) {
-    const size_t cs = q / inner, ij = q - cs * inner;
-    const int j = static_cast<int>(ij / g.nx), i = static_cast<int>(ij - static_cast<size_t>(j) * g.nx);
-    const size_t kc = static_cast<size_t>(j + kGhosts) * g.mx + i + kGhosts;
-    if (g.has_cut && g.vol[kc] <= 0.0) continue;
-    const size_t k = cs * 4 * pl + kc;
-    const double d = g.dt[cs];
-    if (d > 0.0) {
-      double rate;
-      if (!g.has_cut) {
-        rate = wave_bound(Q[k], Q[k + pl], Q[k + 2 * pl], Q[k + 3 * pl], g, g.dx[i + kGhosts], g.dy[j + kGhosts]);
-      } else {
-        // implicit_spectral_rate of a cell of a cut grid (src/implicit2d.h:33-43)
-        const double r = Q[k], mu = Q[k + pl], mv = Q[k + 2 * pl], E = Q[k + 3 * pl];
-        const double u = mu / r, v = mv / r;
-        const double p = pressure(r, mu, mv, E, g.gamma);
-        const double a = sqrt(g.gamma * p / r);
-        const size_t fe = static_cast<size_t>(j) * (g.nx + 1) + i, fn = static_cast<size_t>(j) * g.nx + i;
-        const double wx = g.wax[kc], wy = g.way[kc];
-        const double wall = sqrt(wx * wx + wy * wy);
-        rate = ((fabs(u) + a) * (g.axl[fe + 1] + g.axl[fe]) + (fabs(v) + a) * (g.ayl[fn + g.nx] + g.ayl[fn]) +
-                fabs(u * wx + v * wy) + a * wall) /
-               (2.0 * g.vol[kc]);
-      }
-      const double omega = pseudo / (pseudo + d * rate);
-      for (int v = 0; v < 4; ++v) {
-        const size_t kv = k + v * pl;
-        trial[kv] = Q[kv] + omega * (d * g.R[kv] - (Q[kv] - u[kv]));
+      if (converged) {
+        c->cur = c->qbuf;
+        c->nsteps += 1;
+        c->steps += 1;
+        c->phase = PH_BOUND;
+      } else if (limit) {
+        c->status = 4;
+        c->reason = WHY_MAXITER;
       }
     }
-    if (inadmissible(trial[k], trial[k + pl], trial[k + 2 * pl], trial[k + 3 * pl], g.gamma)) bad = true;
+    if (converged || limit) {
+      if (lane == 0) {
+        c->bad = 0;
+        c->events += 1;
+      }
+      return;
+    }
+  } else if (!g.use_part) {
+    for (int k = lane; k < g.ncase; k += kLanes) g.norm[k] = 0;
   }
-  if (__any(bad) && threadIdx.x % kLanes == 0) atomicOr(&g.ctrl->bad, 1);
-}
-
-// Candidate accepted as the next iterate, or the pseudo CFL halved (12 retries, then 2).
-__global__ __launch_bounds__(kLanes) void k_be_check(Grid g) {
-  Control* c = g.ctrl;
-  if (threadIdx.x != 0 || c->status != RUNNING || c->phase != PH_TRIAL) return;
-  if (c->bad) {
-    c->bad = 0;
+  if (lane != 0) return;
+  c->bad = 0;
+  if (bad) {
     c->iretries += 1;
     c->pretries += 1;
     if (c->pretries > kMaxRetries) {
@@ -1142,12 +1131,13 @@ __global__ __launch_bounds__(kLanes) void k_be_check(Grid g) {
       c->reason = WHY_PSEUDO;
     } else {
       c->pseudo *= 0.5;
+      c->phase = PH_RETRY;
     }
   } else {
     c->qbuf = 3 - c->cur - c->qbuf;
     c->updates += 1;
     c->iter += 1;
-    c->phase = PH_RES;
+    c->phase = PH_UPDATE;
   }
   c->events += 1;
 }
@@ -1496,7 +1486,10 @@ void launch_stage_srd(ugrid_session* s, hipStream_t stream) {
                      dim3(kThreads), 0, stream, g);
 }
 
-// One backward-Euler replay: every phase kernel once, in phase order.
+// One backward-Euler round: the kernels that open a step, then kUpdates pseudo updates.  A step of
+// tens of updates pays the opening kernels' three empty launches once in a round, and at most a round
+// less one of empty updates at its end.
+constexpr int kUpdates = 8;
 int launch_be_round(ugrid_session* s, hipStream_t stream) {
   const Grid& g = s->g;
   const long long inner = static_cast<long long>(g.nx) * g.ny;
@@ -1506,11 +1499,11 @@ int launch_be_round(ugrid_session* s, hipStream_t stream) {
   hipLaunchKernelGGL(k_bound, dim3(per_case * g.ncase), dim3(kThreads), 0, stream, g, per_case, PH_BOUND);
   hipLaunchKernelGGL(k_be_open, dim3(1), dim3(kLanes), 0, stream, g);
   hipLaunchKernelGGL(k_be_copy, dim3(grid_blocks(g, 4 * cells)), dim3(kThreads), 0, stream, g);
-  launch_stage<4>(s, stream);
-  hipLaunchKernelGGL(k_be_decide, dim3(1), dim3(kDecide), 0, stream, g);
-  hipLaunchKernelGGL(k_be_trial, dim3(grid_blocks(g, cells)), dim3(kThreads), 0, stream, g);
-  hipLaunchKernelGGL(k_be_check, dim3(1), dim3(kLanes), 0, stream, g);
-  return 7;
+  for (int u = 0; u < kUpdates; ++u) {
+    launch_stage<4>(s, stream);
+    hipLaunchKernelGGL(k_be_decide, dim3(1), dim3(kDecide), 0, stream, g);
+  }
+  return 3 + 2 * kUpdates;
 }
 
 int launch_trial(ugrid_session* s, hipStream_t stream) {
@@ -1797,7 +1790,6 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
           "hipHostMalloc") ||
       !device_alloc(s, &g.B[0], states, err, err_len) || !device_alloc(s, &g.B[1], states, err, err_len) ||
       !device_alloc(s, &g.B[2], states, err, err_len) || !device_alloc(s, &dxd, g.mx, err, err_len) ||
-      (p.time_integrator == 1 && !device_alloc(s, &g.R, states, err, err_len)) ||
       !device_alloc(s, &g.norm, g.ncase, err, err_len) ||
       !device_alloc(s, &g.part, g.use_part ? g.strips : 1, err, err_len) || !device_alloc(s, &g.initial, g.ncase, err, err_len) ||
       !device_alloc(s, &dyd, g.my, err, err_len) || !device_alloc(s, &rdx, g.mx, err, err_len) ||
@@ -1847,7 +1839,8 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
     release(s);
     return 3;
   }
-  const int trials = g.nx * static_cast<long long>(g.ny) * g.ncase >= (1 << 22) ? 4 : 16;
+  int trials = g.nx * static_cast<long long>(g.ny) * g.ncase >= (1 << 22) ? 4 : 16;
+  if (p.time_integrator == 1) trials /= 4;  // rounds of kUpdates updates
   if (!build_graph(s, trials, err, err_len)) {
     release(s);
     return 3;

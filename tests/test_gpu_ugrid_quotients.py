@@ -105,3 +105,22 @@ def test_downloaded_ghosts(bc, nx, ny):
         inner = s.U.reshape(3, 4, ny + 4, nx + 4)[:, :, 2:-2, 2:-2]
         np.testing.assert_array_equal(inner, ref["u"].reshape(3, 4, ny + 4, nx + 4)[:, :, 2:-2, 2:-2])
         np.testing.assert_array_equal(s.U, ref["u"])
+
+
+@pytest.mark.parametrize("cases", [3, 1023, 1025])  # norms by the strips' partials / by atomics
+def test_many_cases_implicit(cases):
+    """Backward Euler with refused candidates (each formed again from the same iterate) and steps of
+    more updates than one round of launches holds."""
+    s = solver(5, 4, cases, E.FLUX_HLLC)
+    s.par.time_integrator, s.par.cfl, s.par.pseudo_cfl = E.TIME_BACKWARD_EULER, 2.0, 1000.0
+    ref = G.run_implicit(s, 1e300, 2)
+    assert ref["updates"] > 16
+    with s.device_session() as d:
+        status, _ = d.run(1e300, 2)
+        got = d.implicit_stats()
+        d.pull()
+    assert status == ref["status"]
+    for key in ("updates", "retries", "checks", "initial_defect", "final_defect"):
+        assert got[key] == ref[key], key
+    np.testing.assert_array_equal(s.U, ref["u"])
+    np.testing.assert_array_equal(s.t, ref["t"])
