@@ -19,8 +19,9 @@
 //     ghost (negation is exact).
 //   * the RK update, the admissibility test of the candidate and, in the last stage, the
 //     candidate's wave-speed bound for the next step's dt are fused into the same pass.  A
-//     one-wave kernel after the last stage commits or rejects the trial for all cases: t += dt, step counters, buffer swap (U[cur] and the other buffer alternate, so no
-//     accept copy), next dt from the bound, or dt halving and the 12-retry limit.
+//     one-block kernel after the last stage reduces the strips' bounds and commits or rejects the
+//     trial for all cases: t += dt, step counters, buffer swap (U[cur] and the other buffer
+//     alternate, so no accept copy), next dt from the bound, or dt halving and the 12-retry limit.
 //   * a trial is four launches; the host replays a graph of several trials and polls the
 //     control record between replays.
 // The arithmetic of every formula follows the reference's GPU kernels operation for operation
@@ -59,7 +60,7 @@ constexpr int kPrechecks = 8;
 enum : int { BC_PERIODIC = 0, BC_TRANSMISSIVE = 1, BC_REFLECT = 2 };
 enum : int { RUNNING = -1 };
 // Backward-Euler phases of a physical step (each kernel of the replayed sequence acts only in its
-// phase; the one-wave decision kernels move the phase).
+// phase; the one-block decision kernels move the phase).
 enum : int { PH_BOUND = 0, PH_COPY = 1, PH_UPDATE = 2, PH_RETRY = 3 };
 // Why a backward-Euler run stopped with 2, 3 or 4.
 enum : int { WHY_NONE = 0, WHY_INITIAL = 1, WHY_PSEUDO = 2, WHY_DEFECT = 3, WHY_MAXITER = 4, WHY_DT = 5 };
