@@ -13,6 +13,8 @@ import pytest
 from oracle import pygrid as G
 from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import euler2d as E
 
+from .grid_cases import cut_body
+
 pytestmark = pytest.mark.gpu
 
 
@@ -124,3 +126,15 @@ def test_many_cases_implicit(cases):
         assert got[key] == ref[key], key
     np.testing.assert_array_equal(s.U, ref["u"])
     np.testing.assert_array_equal(s.t, ref["t"])
+
+
+@pytest.mark.parametrize("halvings", [1, 6, 7, 8, 9, 12, 13])  # within, at and past one pre-check's steps, and too many
+@pytest.mark.parametrize("flux", [E.FLUX_HLLC, E.FLUX_AUSMPUP])
+def test_halvings_of_a_step_on_a_cut_grid(flux, halvings):
+    par = E.params2d_default()
+    par.limiter, par.flux = E.LIM_FIRST_ORDER, flux
+    par.dt_fixed = 2.0 ** (halvings - 11)  # 2^-11 is admissible in the smallest cut cells
+    s, _, _ = cut_body("circle", 52, 40, par, shock=-0.6)
+    ref = G.run(s, 1e300, 1)
+    assert ref["nreject"] == halvings and ref["status"] == (2 if halvings == 13 else 1)
+    check(s, 1)
