@@ -1377,8 +1377,8 @@ struct ugrid_session {
   std::vector<double> mco;   // host copy of the reference Mach numbers
   Control* host_ctrl = nullptr;  // pinned mirror of the control record
   hipStream_t stream = nullptr;
-  hipGraphExec_t exec = nullptr;
-  int graph_trials = 0;
+  hipGraphExec_t exec = nullptr;      // trials, or backward-Euler rounds of kUpdates updates
+  hipGraphExec_t exec_one = nullptr;  // backward-Euler rounds of one update
   std::vector<void*> owned;
 };
 
@@ -1410,7 +1410,8 @@ bool device_alloc(ugrid_session* s, T** p, size_t count, char* err, size_t len) 
 
 void release(ugrid_session* s) {
   if (!s) return;
-  if (s->exec) (void)hipGraphExecDestroy(s->exec);
+  for (hipGraphExec_t e : {s->exec, s->exec_one})
+    if (e) (void)hipGraphExecDestroy(e);
   for (void* p : s->owned) (void)hipFree(p);
   if (s->host_ctrl) (void)hipHostFree(s->host_ctrl);
   if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -1501,24 +1502,30 @@ void launch_stage_srd(ugrid_session* s, hipStream_t stream) {
                      dim3(kThreads), 0, stream, g);
 }
 
-// One backward-Euler round: the kernels that open a step, then kUpdates pseudo updates.  A step of
-// tens of updates pays the opening kernels' three empty launches once in a round, and at most a round
-// less one of empty updates at its end.
+// One backward-Euler round: the kernels that open a step, then `updates` pseudo updates.  A launch that
+// finds nothing to do costs about 3.5 us.  A step of tens of updates wants long rounds: with kUpdates it
+// pays the three opening kernels once in eight updates, and at most a round less one of empty updates
+// at its end.  A step that needs kFewChecks updates or fewer (a nearly steady flow) wastes less in
+// rounds of one: 3 launches for each update but the first instead of 2 for each one missing of eight.
+// One case of 64 x 64 whose steps converge at their first check takes 45 us a step in long rounds and 24
+// in rounds of one, 8 cases of 256 x 256 99 and 59.  The host chooses by the updates a step of the last
+// replay.
 constexpr int kUpdates = 8;
-int launch_be_round(ugrid_session* s, hipStream_t stream) {
+constexpr int kFewChecks = 3;
+int launch_be_round(ugrid_session* s, hipStream_t stream, int updates) {
   const Grid& g = s->g;
   const long long inner = static_cast<long long>(g.nx) * g.ny;
-  const int per_case = static_cast<int>(
-      std::max<long long>(1, std::min<long long>((inner + kThreads - 1) / kThreads, 2048 / g.ncase)));
+  const long long blocks = (inner + 4 * kThreads - 1) / (4 * kThreads);
+  const int per_case = static_cast<int>(blocks < 1 ? 1 : blocks > 256 ? 256 : blocks);
   const size_t cells = static_cast<size_t>(inner) * g.ncase;
   hipLaunchKernelGGL(k_bound, dim3(per_case * g.ncase), dim3(kThreads), 0, stream, g, per_case, PH_BOUND);
   hipLaunchKernelGGL(k_be_open, dim3(1), dim3(kLanes), 0, stream, g);
   hipLaunchKernelGGL(k_be_copy, dim3(grid_blocks(g, 4 * cells)), dim3(kThreads), 0, stream, g);
-  for (int u = 0; u < kUpdates; ++u) {
+  for (int u = 0; u < updates; ++u) {
     launch_stage<4>(s, stream);
     hipLaunchKernelGGL(k_be_decide, dim3(1), dim3(kDecide), 0, stream, g);
   }
-  return 3 + 2 * kUpdates;
+  return 3 + 2 * updates;
 }
 
 int launch_trial(ugrid_session* s, hipStream_t stream) {
@@ -1529,16 +1536,13 @@ int launch_trial(ugrid_session* s, hipStream_t stream) {
   return 4;
 }
 
-bool build_graph(ugrid_session* s, int trials, char* err, size_t len) {
-  if (s->exec) {
-    (void)hipGraphExecDestroy(s->exec);
-    s->exec = nullptr;
-  }
+// `count` trials, or backward-Euler rounds of `updates` updates, as a graph.
+bool build_graph(ugrid_session* s, int count, int updates, hipGraphExec_t* exec, char* err, size_t len) {
   hipGraph_t graph = nullptr;
   if (!ok(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal), err, len, "begin capture")) return false;
-  for (int k = 0; k < trials; ++k) {
+  for (int k = 0; k < count; ++k) {
     if (s->par.time_integrator == 1)
-      launch_be_round(s, s->stream);
+      launch_be_round(s, s->stream, updates);
     else
       launch_trial(s, s->stream);
   }
@@ -1548,11 +1552,9 @@ bool build_graph(ugrid_session* s, int trials, char* err, size_t len) {
     if (graph) (void)hipGraphDestroy(graph);
     return false;
   }
-  const hipError_t inst = hipGraphInstantiate(&s->exec, graph, nullptr, nullptr, 0);
+  const hipError_t inst = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
-  if (!ok(inst, err, len, "graph instantiate")) return false;
-  s->graph_trials = trials;
-  return true;
+  return ok(inst, err, len, "graph instantiate");
 }
 
 // Cut-cell arrays of the device: per-cell data, apertures, and the SRD lists (members of each
@@ -1854,9 +1856,10 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
     release(s);
     return 3;
   }
-  int trials = g.nx * static_cast<long long>(g.ny) * g.ncase >= (1 << 22) ? 4 : 16;
-  if (p.time_integrator == 1) trials /= 4;  // rounds of kUpdates updates
-  if (!build_graph(s, trials, err, err_len)) {
+  const int trials = g.nx * static_cast<long long>(g.ny) * g.ncase >= (1 << 22) ? 4 : 16;
+  const bool implicit = p.time_integrator == 1;
+  if (!build_graph(s, implicit ? trials / 4 : trials, kUpdates, &s->exec, err, err_len) ||
+      (implicit && !build_graph(s, trials / 2, 1, &s->exec_one, err, err_len))) {
     release(s);
     return 3;
   }
@@ -1896,6 +1899,9 @@ extern "C" int ugrid_run(ugrid_session* s, double tend, int64_t maxsteps, ugrid_
   // phase change), so it must move the event count; a replay that does not is reported, not
   // waited on.
   long long progress = -1;
+  // Backward Euler: steps, and update kernels that they used, up to the last poll; the first round of a
+  // run is launched by itself, and those after it by what it showed.
+  long long steps = 0, used = 0;
   for (;;) {
     if (!ok(hipMemcpyAsync(s->host_ctrl, g.ctrl, sizeof(Control), hipMemcpyDeviceToHost, s->stream), err, err_len,
             "control copy") ||
@@ -1904,8 +1910,21 @@ extern "C" int ugrid_run(ugrid_session* s, double tend, int64_t maxsteps, ugrid_
     if (s->host_ctrl->status != RUNNING) break;
     const long long now = s->host_ctrl->events;
     if (now == progress) return fail(err, err_len, "ugrid_run: device step control made no progress");
+    const bool first = progress == -1;
     progress = now;
-    if (!ok(hipGraphLaunch(s->exec, s->stream), err, err_len, "trial graph")) return 3;
+    hipGraphExec_t exec = s->exec;
+    if (implicit) {
+      const long long made = s->host_ctrl->nsteps - steps, tries = s->host_ctrl->checks + s->host_ctrl->iretries - used;
+      steps += made;
+      used += tries;
+      if (first) {
+        launch_be_round(s, s->stream, kUpdates);
+        if (!ok(hipGetLastError(), err, err_len, "round launch")) return 3;
+        continue;
+      }
+      if (made > 0 && tries <= kFewChecks * made) exec = s->exec_one;
+    }
+    if (!ok(hipGraphLaunch(exec, s->stream), err, err_len, "trial graph")) return 3;
   }
   const Control& c = *s->host_ctrl;
   if (meta) {

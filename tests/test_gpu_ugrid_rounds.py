@@ -1,0 +1,64 @@
+"""Backward-Euler steps of few and of many pseudo updates in one run: the host replays short or long
+rounds by what the last replay's steps needed, which changes no decision, and a step that converges
+at its first check is not held up by the updates that it does not need.
+"""
+import time
+
+import numpy as np
+import pytest
+
+from oracle import pygrid as G
+from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import euler2d as E
+
+pytestmark = pytest.mark.gpu
+
+
+def pulse(nx, ny, amplitude, integrator, cfl=4.0, tol=1e-4, cases=2):
+    """A density pulse that a supersonic stream carries out of the domain."""
+    par = E.params2d_default()
+    par.limiter, par.time_integrator, par.cfl, par.pseudo_cfl = E.LIM_FIRST_ORDER, integrator, cfl, 4.0
+    par.implicit_rtol = par.implicit_atol = tol
+    s = E.Solver2D(nx, ny, 0.0, 1.0, 0.0, ny / nx, cases, par)
+    x = s.grid.xc[2:-2][None, :]
+    for c in range(cases):
+        s.set_primitive_field(c, 1.0 + amplitude * (c + 1) * np.exp(-100.0 * (x - 0.5) ** 2), 1.5, 0.0, 1.0)
+    return s
+
+
+@pytest.mark.parametrize("cfl, tol, per_step", [(4.0, 1e-4, {0, 1, 2, 4, 25, 70}), (1.0, 1e-3, {2, 3})])
+@pytest.mark.parametrize("runs", [(40,), (1, 21, 3, 15)])
+def test_steps_of_few_and_many_updates(cfl, tol, per_step, runs):
+    s = pulse(24, 3, 0.2, E.TIME_BACKWARD_EULER, cfl, tol)
+    refs = [G.run_implicit(s, 1e300, n)["updates"] for n in range(1, 41)]
+    assert per_step <= set(np.diff([0] + refs))
+    ref = G.run_implicit(s, 1e300, 40)
+    with s.device_session() as d:
+        for steps in runs:
+            status, message = d.run(1e300, steps)
+        d.pull()
+        got = d.implicit_stats()
+    assert status == ref["status"] == 1, message
+    for key in ("updates", "retries", "checks", "initial_defect", "final_defect"):
+        assert got[key] == ref[key], key
+    for have, want in ((s.U, ref["u"]), (s.t, ref["t"]), (s.dt, ref["dt"])):
+        np.testing.assert_array_equal(have, want)
+
+
+def test_step_that_converges_at_once_is_short():
+    """A uniform state's step is five dependent launches, an SSP-RK3 step four (stages that march three
+    rows as the update does): 24 against 22 us on one case of 64 x 64, 45 where a step's round holds
+    eight updates."""
+    best = {}
+    for integrator in (E.TIME_BACKWARD_EULER, E.TIME_SSP_RK3):
+        with pulse(64, 64, 0.0, integrator, cases=1).device_session() as d:
+            d.run(1e300, 20)
+            for _ in range(8):
+                t0 = time.perf_counter()
+                status, _ = d.run(1e300, 200)
+                best[integrator] = min(best.get(integrator, 1e9), time.perf_counter() - t0)
+                assert status == 1
+            if integrator == E.TIME_BACKWARD_EULER:
+                assert d.implicit_stats()["updates"] == 0
+    ratio = best[E.TIME_BACKWARD_EULER] / best[E.TIME_SSP_RK3]
+    print("us a step", {k: round(v / 200 * 1e6, 2) for k, v in best.items()}, "ratio", ratio, flush=True)
+    assert ratio < 1.6
