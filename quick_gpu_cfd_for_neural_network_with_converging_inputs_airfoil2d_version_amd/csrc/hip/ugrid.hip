@@ -1967,8 +1967,8 @@ extern "C" int ugrid_download(ugrid_session* s, double* u, uint64_t u_len, doubl
   const size_t bytes = s->states * sizeof(double);
   // Once a step has begun, the ghosts are a boundary fill that the device makes in the accepted
   // state's own buffer (its kernels never read ghost cells): one copy, instead of a second state
-  // beside it and two passes of the host over both (8 cases of 1024 x 1024: 123 -> 15 ms with the
-  // mirror's pull in place).
+  // beside it and two passes of the host over both (8 cases of 1024 x 1024: the Python pull, which
+  // copies the state once more on the host, 123 -> 19 ms).
   if (u && c.ghost_from != 0 && g.nx >= 2 && g.ny >= 2 && g.my <= 65535 && 4LL * g.ncase <= 65535) {
     const double* from = c.ghost_from == 1 ? g.B[c.cur] : g.B[c.cur ^ 1];
     hipLaunchKernelGGL(k_fill_ghosts, dim3(g.my, 4 * g.ncase), dim3(kThreads), 0, s->stream, g, from, g.B[c.cur]);
