@@ -98,7 +98,7 @@ struct Grid {
   const double* dy;    // my
   const double* rdx;   // recip() of every width
   const double* rdy;
-  int plain;           // widths, gamma - 1 and reference Mach numbers are plain (see `recip`)
+  int plain;           // widths, gamma - 1 and AUSM+-up's reference Mach numbers are plain (see `recip`)
   const double* mco;   // ncase
   // State buffers: B[0] and B[1] alternate as accepted state and RK candidate, B[2] holds the
   // second RK stage; backward Euler rotates all three (accepted state, iterate, candidate).
@@ -171,7 +171,7 @@ struct Flux {
 // (PLAIN false) the compiler's division and square root are used.
 //
 // Plain (`plain_state`): density and pressure in (2^-100, 2^100), energy below 2^100, which bounds
-// the velocities through p > 0; cell widths, gamma - 1 and the reference Mach numbers likewise
+// the velocities through p > 0; cell widths, gamma - 1 and AUSM+-up's reference Mach numbers likewise
 // (Grid::plain).  Every divisor the kernels form is then a normal number in (2^-400, 2^400).  A
 // numerator may be arbitrarily small where a velocity or a flux difference is (zero and rounding
 // noise ahead of a wave): such quotients are formed of the numerator times 2^200 (`quot_scaled`),
@@ -1797,7 +1797,7 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   bool plain = plain_value(p.gamma - 1.0) && plain_value(p.gamma);
   for (int k = 0; k < g.mx; ++k) plain = plain && plain_value(setup->dx[k]);
   for (int k = 0; k < g.my; ++k) plain = plain && plain_value(setup->dy[k]);
-  for (int c = 0; c < g.ncase; ++c) plain = plain && plain_value(mco[c]);
+  for (int c = 0; g.ausm && c < g.ncase; ++c) plain = plain && plain_value(mco[c]);  // (HLLC reads none)
   g.plain = plain ? 1 : 0;
 
   double *dxd = nullptr, *dyd = nullptr, *rdx = nullptr, *rdy = nullptr, *mcod = nullptr;
