@@ -462,13 +462,14 @@ def main():
     else:
         tile, tile_times = AT.pick_tile(meshes, params, states, precision=32, trials=30, warmup=10)
     log("tile us/step: " + ", ".join(f"{t}: {s * 1e6:.1f}" for t, s in tile_times.items()) + f" -> {tile}")
-    # Few-slot launch shape (two flux threads per cell once at most few_slots slots run).
+    # Few-slot launch shape (more flux threads per cell once at most few_slots slots run).
     if args.few_slots < 0:
-        few_slots, few_times = AT.pick_few_slots(meshes, params, states, precision=32, tile=tile)
-        log("few-slot trial us (1 / 2 flux threads per cell): " +
-            ", ".join(f"{k} running: {a} / {b}" for k, (a, b) in sorted(few_times.items())) + f" -> {few_slots}")
+        few_slots, few_spread, few_times = AT.pick_few_shape(meshes, params, states, precision=32, tile=tile)
+        log("few-slot trial us by flux threads per cell: " +
+            ", ".join(f"{k} running: {t}" for k, t in sorted(few_times.items())) +
+            f" -> {few_spread} at {few_slots} and fewer")
     else:
-        few_slots, few_times = args.few_slots, {}
+        few_slots, few_spread, few_times = args.few_slots, 2, {}
 
     # 2. Timed steps of the batch: exactly --steps graph replays after --warmup.
     with B.Batch.of_meshes(meshes, params, states, precision=32, tile=tile, graph=args.graph) as b:
@@ -510,8 +511,8 @@ def main():
     if args.solve:
         # 3. Batched FP32 steady solve of the whole batch (the headline value).
         with B.Batch.of_meshes(meshes, params, states, precision=32, tile=tile) as b:
-            if tile * 2 <= 256 and few_slots > 0:
-                b.set_launch_shape(1, few_slots, 2)  # two flux threads per cell once few slots run
+            if few_slots > 0:
+                b.set_launch_shape(0, few_slots, few_spread)
             t0 = time.perf_counter()
             res32 = b.solve(cases, mode="steady", budget=args.budget)
             wall32 = time.perf_counter() - t0
@@ -681,8 +682,8 @@ def main():
             "batch": args.batch, "seed": args.seed, "mesh": "LF2 (6 levels, wall h/c 1/128)",
             "cells_total": int(sum(cells)), "cells_min": int(min(cells)), "cells_max": int(max(cells)),
             "tile": tile, "parallelism": "single GPU",
-            "few_slot_flux_threads_per_cell": {"slots": few_slots, "threads": 2, "probe_us": few_times}
-            if tile * 2 <= 256 and few_slots > 0 else None,
+            "few_slot_flux_threads_per_cell": {"slots": few_slots, "threads": few_spread, "probe_us": few_times}
+            if few_slots > 0 else None,
         },
         "roofline": {
             "bound": "hbm", "achieved": round(achieved, 1), "peak": RL.HBM_PEAK_GBPS, "unit": "GB/s",

@@ -331,12 +331,16 @@ int amr_batch_advance(amr_batch* b, int32_t until, double wall_budget_seconds, a
 /* Exactly `trials` trials, then one poll. */
 int amr_batch_run(amr_batch* b, int32_t trials, amr_slot_state* states, char* err, size_t err_len);
 /* Launch shape of the trials (no counterpart in the reference; a batch tuning knob): the flux
- * launches run flux_spread threads per cell (1 or 2; tile * spread <= 256), and while at most
+ * launches run flux_spread threads per cell (1 to 3; tile * spread <= 512), and while at most
  * few_slots slots are running (0: never) few_flux_spread instead, so that a nearly drained batch,
- * whose trials are bound by latency, spreads each tile's face items over more threads.  Results
- * are bitwise independent of the shape.  Recaptures the trial graphs.  0 ok, 1 invalid or error. */
+ * whose trials are bound by latency, spreads each tile's face items over more threads.  A spread of
+ * 0 is the one that the arena chose by its size when it was made, which it runs until this call.
+ * Results are bitwise independent of the shape.  Recaptures the trial graphs.  0 ok, 1 invalid or
+ * error. */
 int amr_batch_set_launch_shape(amr_batch* b, int32_t flux_spread, int32_t few_slots, int32_t few_flux_spread, char* err,
                                size_t err_len);
+/* The launch shape in use: shape[0..2] = flux_spread, few_slots, few_flux_spread (never 0). */
+int amr_batch_launch_shape(const amr_batch* b, int32_t* shape);
 /* Slot states of the last poll (no device access). */
 int amr_batch_slots(const amr_batch* b, amr_slot_state* states);
 int32_t amr_batch_size(const amr_batch* b);

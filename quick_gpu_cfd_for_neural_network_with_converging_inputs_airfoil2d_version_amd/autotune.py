@@ -14,11 +14,15 @@ bitwise identical between runs at the same tile, and within the FP64/FP32 tolera
 tiles (the monitor's block partial sums are the only tile-dependent reduction order).
 
 The second choice is the few-slot launch shape (`Batch.set_launch_shape`): when few slots of a
-closed batch are still running, each trial is bound by latency and two threads per cell in the
-flux launches shorten it; with many running it is slower (fewer blocks per CU).  The tuner times
-trials with k = 32, 16, 8 and 2 running slots at one and two threads per cell and keeps the
-largest k at and below which two threads win every probe (0: never).  Results are bitwise
-independent of both choices at a given tile.
+closed batch are still running, each trial is bound by latency and more threads per cell in the
+flux launches shorten it; with many running they are slower (fewer blocks per CU).  The tuner times
+trials with k = 32, 16, 8 and 2 running slots at the spread that the arena chose by its size and at
+every larger one that the tile admits, and takes the one that wins at and below the largest k (0:
+none wins, or the arena's own spread is the largest there is).  256 LF2 meshes, FP32, tile 128, us a
+trial at one / two / three threads: 2 running 66.2 / 61.4 / 57.5, 8: 69.3 / 64.5 / 72.3, 16: 82.6 /
+77.4 / 114, 32: 101 / 117 / 167, so two threads from 16 slots down (the blocks of ended slots, which
+the others wait behind, hold as many threads).  Results are bitwise independent of both choices at a
+given tile.
 
 Results are cached per (precision, slot count, total cells rounded to 1%, feature set) for
 the life of the process.
@@ -70,26 +74,30 @@ def pick_tile(meshes, params, states, precision: int = 32, tiles=TILES, trials: 
 
 
 FEW_PROBES = (32, 16, 8, 2)
+MAX_BLOCK = 512  # threads of the largest flux block
 
 
-def pick_few_slots(meshes, params, states, precision: int, tile: int, probes=FEW_PROBES, seconds: float = 0.25,
-                   warmup: int = 10) -> tuple[int, dict]:
-    """(few_slots for two flux threads per cell, {k: (us per trial at 1, at 2)}) at this tile;
-    (0, {}) when the tile has no room for two threads per cell (tile 256)."""
-    if tile * 2 > 256 or len(meshes) < 2:
-        return 0, {}
+def pick_few_shape(meshes, params, states, precision: int, tile: int, probes=FEW_PROBES, seconds: float = 0.25,
+                   warmup: int = 10, spreads=(2, 3)) -> tuple[int, int, dict]:
+    """(few_slots, few_flux_spread, {k: {threads per cell: us per trial}}) at this tile, for
+    `Batch.set_launch_shape(0, few_slots, few_flux_spread)`; (0, 0, {}) when no spread of `spreads` is
+    larger than the arena's own."""
+    if len(meshes) < 2:
+        return 0, 0, {}
     feats = B.union([B.capacity(m)[1] for m in meshes])
-    key = ("few",) + _key(meshes, precision, feats) + (tile,)
+    key = ("few", tuple(spreads)) + _key(meshes, precision, feats) + (tile,)
     if key in _CACHE:
         return _CACHE[key]
     n = len(meshes)
     out = {}
     with B.Batch.of_meshes(meshes, params, states, precision=precision, tile=tile) as b:
+        own = b.launch_shape()[0]
+        tried = [own] + [s for s in spreads if s > own and tile * s <= MAX_BLOCK]
         b.set_targets(1e30)
         b.run(warmup)
-        for k in sorted({min(k, n) for k in probes}, reverse=True):
-            per = []
-            for spread in (1, 2):
+        for k in sorted({min(k, n) for k in probes}, reverse=True) if len(tried) > 1 else ():
+            out[k] = {}
+            for spread in tried:
                 b.set_launch_shape(spread, 0, spread)
                 b.set_targets([1e30] * k + [0.0] * (n - k))
                 b.run(warmup)
@@ -98,16 +106,36 @@ def pick_few_slots(meshes, params, states, precision: int, tile: int, probes=FEW
                 b.advance("all", budget=seconds)
                 elapsed = time.perf_counter() - t0
                 trials = (sum(s["steps"] + s["rejected"] for s in b.states()[:k]) - before) / k
-                per.append(elapsed / max(trials, 1.0) * 1e6)
-            out[k] = (round(per[0], 1), round(per[1], 1))
-    few = choose_few(out)
-    _CACHE[key] = (few, out)
-    return few, out
+                out[k][spread] = round(elapsed / max(trials, 1.0) * 1e6, 1)
+    few, spread = choose_few_shape(out)
+    _CACHE[key] = (few, spread, out)
+    return few, spread, out
+
+
+def pick_few_slots(meshes, params, states, precision: int, tile: int, probes=FEW_PROBES, seconds: float = 0.25,
+                   warmup: int = 10) -> tuple[int, dict]:
+    """(few_slots for two flux threads per cell, {k: (us per trial at the arena's own, at two)}) at this
+    tile; (0, {}) when the arena runs two or more by itself."""
+    few, _, out = pick_few_shape(meshes, params, states, precision, tile, probes, seconds, warmup, (2,))
+    return few, {k: (t[min(t)], t[2]) for k, t in out.items()}
+
+
+def choose_few_shape(probes: dict) -> tuple[int, int]:
+    """(few_slots, threads per cell) from {running slots: {threads per cell: us per trial}}, the smallest
+    spread of each being the arena's own: the spread that beats it up to the most slots, of two alike the
+    faster with the fewest; (0, 0) when none beats it."""
+    if not probes:
+        return 0, 0
+    fewest = probes[min(probes)]
+    own = min(fewest)
+    found = [(choose_few({k: (t[own], t[s]) for k, t in probes.items()}), -t, s) for s, t in fewest.items() if s != own]
+    few, _, spread = max(found, default=(0, 0, 0))
+    return (few, spread) if few else (0, 0)
 
 
 def choose_few(probes: dict) -> int:
-    """From {running slots: (us per trial at one, at two threads per cell)}: the largest k such
-    that two threads win at k and at every smaller probe (0 if they lose at the smallest)."""
+    """From {running slots: (us per trial at few, at more threads per cell)}: the largest k such
+    that more threads win at k and at every smaller probe (0 if they lose at the smallest)."""
     few = 0
     for k in sorted(probes):
         if probes[k][1] < probes[k][0]:

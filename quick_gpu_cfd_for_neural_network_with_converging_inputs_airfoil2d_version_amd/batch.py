@@ -166,12 +166,19 @@ class Batch:
         self._check(self._lib.amr_batch_run(self.handle, trials, self._state_buf, err, N.ERR_LEN), err)
         return _states(self._state_buf)
 
-    def set_launch_shape(self, flux_spread: int = 1, few_slots: int = 0, few_flux_spread: int = 1) -> None:
-        """Threads per cell of the flux launches, and the spread used while at most `few_slots`
-        slots run (latency-bound trials); results are bitwise independent of the shape."""
+    def set_launch_shape(self, flux_spread: int = 0, few_slots: int = 0, few_flux_spread: int = 0) -> None:
+        """Threads per cell of the flux launches (1 to 3, at most 512 threads per block), and the spread
+        used while at most `few_slots` slots run (latency-bound trials); 0: what the arena chose by its
+        size when it was made.  Results are bitwise independent of the shape."""
         err = N.err_buffer()
         self._check(self._lib.amr_batch_set_launch_shape(self.handle, flux_spread, few_slots, few_flux_spread, err,
                                                           N.ERR_LEN), err)
+
+    def launch_shape(self) -> tuple[int, int, int]:
+        """(threads per cell, few_slots, threads per cell while at most few_slots slots run) in use."""
+        shape = (C.c_int32 * 3)()
+        self._lib.amr_batch_launch_shape(self.handle, shape)
+        return tuple(shape)
 
     def states(self) -> list[dict]:
         self._lib.amr_batch_slots(self.handle, self._state_buf)

@@ -73,6 +73,10 @@ constexpr int kItemInfoMask = 15;
 // 699, 705, 683, 690 and 691 us per batch step (one chunk round for most tiles against losing a
 // block per CU); a stage chunk of 11/4 gains nothing, 3 loses 13 us per stage pass.
 __host__ __device__ constexpr int item_round(int tile) { return tile * 5 / 2; }
+// Threads per cell of the flux launches: one to three, in blocks of at most 512 threads.
+__host__ __device__ constexpr bool flux_spread_ok(int tile, int spread) {
+  return spread >= 1 && spread <= 3 && tile * spread <= 512;
+}
 // With three threads per cell a chunk is two rounds: such launches leave LDS to spare, and a tile of more
 // than 5/2 items per cell (in one of ten tiles of an LF2 mesh) evaluated the rest after a barrier, 3 us
 // of a launch's 11.  A cell sums its faces round by round whatever the chunk, so the bits stay.

@@ -46,6 +46,7 @@ struct amr_batch {
   // with few_spread threads per cell in the flux launches (the per-trial latency then dominates,
   // and spreading a tile's face items shortens each flux launch); otherwise spread.
   int spread = 1, few_slots = 0, few_spread = 1;
+  int own_spread = 1;  // the arena's own choice, which it starts with
   std::vector<hipGraphExec_t> execs_few, execs_batch_few;
   Control* host_control = nullptr;  // pinned, n slots
   double* host_targets = nullptr;   // pinned, n slots
@@ -280,7 +281,7 @@ int capture_all(amr_batch* b, char* err, size_t err_len) {
 // Stream, pinned control mirrors, optional graph; the arena is already built.
 int finish_setup(amr_batch* b, Clock::time_point t0, char* err, size_t err_len) {
   const int n = b->n;
-  b->spread = b->arena->flux_spread();
+  b->own_spread = b->spread = b->few_spread = b->arena->flux_spread();
   if (!checked(hipHostMalloc(reinterpret_cast<void**>(&b->host_control), n * sizeof(Control), hipHostMallocDefault),
                err, err_len, "AMR pinned control") ||
       !checked(hipHostMalloc(reinterpret_cast<void**>(&b->host_targets), n * sizeof(double), hipHostMallocDefault), err,
@@ -540,10 +541,11 @@ int amr_batch_run(amr_batch* b, int32_t trials, amr_slot_state* states, char* er
 
 int amr_batch_set_launch_shape(amr_batch* b, int32_t flux_spread, int32_t few_slots, int32_t few_flux_spread, char* err,
                                size_t err_len) {
-  const auto ok_spread = [&](int s) { return s == 1 || s == 2; };
-  if (!b || !ok_spread(flux_spread) || !ok_spread(few_flux_spread) || few_slots < 0 ||
-      b->options.tile * std::max(flux_spread, few_flux_spread) > 256)
-    return fail(err, err_len, "invalid AMR launch shape (threads per cell 1 or 2, at most 256 per block)");
+  if (b && flux_spread == 0) flux_spread = b->own_spread;
+  if (b && few_flux_spread == 0) few_flux_spread = b->own_spread;
+  const auto ok_spread = [&](int s) { return hipamr::flux_spread_ok(b->options.tile, s); };
+  if (!b || !ok_spread(flux_spread) || !ok_spread(few_flux_spread) || few_slots < 0)
+    return fail(err, err_len, "invalid AMR launch shape (threads per cell 1 to 3, at most 512 per block; 0: the arena's own)");
   if (!checked(hipStreamSynchronize(b->stream), err, err_len, "AMR launch shape")) return 1;
   for (hipStream_t s : b->sides)
     if (!checked(hipStreamSynchronize(s), err, err_len, "AMR launch shape")) return 1;
@@ -553,6 +555,14 @@ int amr_batch_set_launch_shape(amr_batch* b, int32_t flux_spread, int32_t few_sl
   b->few_spread = few_flux_spread;
   if (b->options.graph) return capture_all(b, err, err_len);
   b->arena->set_flux_spread(flux_spread);
+  return 0;
+}
+
+int amr_batch_launch_shape(const amr_batch* b, int32_t* shape) {
+  if (!b || !shape) return 1;
+  shape[0] = b->spread;
+  shape[1] = b->few_slots;
+  shape[2] = b->few_spread;
   return 0;
 }
 

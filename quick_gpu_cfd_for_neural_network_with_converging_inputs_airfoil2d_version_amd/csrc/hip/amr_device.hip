@@ -92,7 +92,7 @@ inline int round_up(int n, int tile) { return (n + tile - 1) / tile * tile; }
 int flux_spread_for(int tiles, int tile, int precision) {
   const int resident = 256 * 4 * (precision == 64 ? 3 : 7);  // waves that the flux kernels' registers admit
   int spread = 3;
-  while (spread > 1 && (tile * spread > 512 || static_cast<long long>(tiles) * (tile / 64) * spread > resident))
+  while (spread > 1 && (!flux_spread_ok(tile, spread) || static_cast<long long>(tiles) * (tile / 64) * spread > resident))
     --spread;
   return spread;
 }
@@ -1000,7 +1000,7 @@ class DeviceArena final : public Arena {
   }
   int launch_prims(hipStream_t s) override { return hipamr::launch_prims<T>(ptrs_, s, nullptr); }
   bool set_flux_spread(int spread) override {
-    if (spread < 1 || spread > 3 || tile_ * spread > 512) return false;  // launch bound
+    if (!flux_spread_ok(tile_, spread)) return false;  // launch bound
     ptrs_.flux_spread = spread;
     return true;
   }

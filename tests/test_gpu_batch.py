@@ -11,6 +11,7 @@ import numpy as np
 import pytest
 
 from oracle import pyoracle as O
+from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import autotune as AT
 from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import batch as B
 from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd.session import BackendError, Session
 
@@ -175,6 +176,46 @@ def test_launch_shapes_change_no_bit(precision):
     with B.Batch.of_meshes([items[0][0]], [items[0][1]], [items[0][2]], precision=precision, tile=128) as b:
         with pytest.raises(BackendError):
             b.set_launch_shape(1, 4, 4)  # four threads per cell
+
+
+@pytest.mark.parametrize("precision", [32, 64])
+def test_every_launch_shape_of_the_arena(precision):
+    """The launch-shape call takes every shape that an arena starts with, up to 512 threads per block, and
+    gives its own choice back: same bits at each, the rest refused and nothing changed by it."""
+    case, mesh, params = case_mesh("G0002", "LF1")
+    u0 = mesh.initialize(params, case.freestream)
+    for tile, own, shapes, refused in ((64, 3, ((3, 0, 3), (1, 1, 3), (2, 2, 1), (0, 1, 1)), ((4, 0, 1), (-1, 0, 1), (1, -1, 1))),
+                                       (128, 3, ((3, 0, 3), (1, 1, 3)), ((1, 1, 4),)),
+                                       (256, 2, ((2, 0, 2), (1, 1, 2)), ((3, 0, 1), (1, 1, 3)))):
+        with B.Batch.of_meshes([mesh] * 2, [params] * 2, [u0] * 2, precision=precision, tile=tile) as b:
+            assert b.launch_shape() == (own, 0, own)
+            b.set_targets([0.004, 0.006])
+            assert b.advance("all") == 0
+            ref = [b.download(k) for k in range(2)]
+        for shape in shapes:
+            print(precision, tile, shape, flush=True)
+            with B.Batch.of_meshes([mesh] * 2, [params] * 2, [u0] * 2, precision=precision, tile=tile) as b:
+                b.set_launch_shape(*shape)
+                assert b.launch_shape() == (shape[0] or own, shape[1], shape[2] or own)
+                for bad in refused:
+                    with pytest.raises(BackendError, match="launch shape"):
+                        b.set_launch_shape(*bad)
+                b.set_targets([0.004, 0.006])
+                assert b.advance("all") == 0
+                for k in range(2):
+                    u, meta = b.download(k)
+                    assert meta == ref[k][1] and np.array_equal(u, ref[k][0]), (tile, shape, k)
+                b.set_launch_shape()
+                assert b.launch_shape() == (own, 0, own)
+
+
+def test_autotuned_shape_of_a_small_arena_keeps_its_own():
+    """An arena that runs three threads per cell by itself has no few-slot shape to switch to."""
+    case, mesh, params = case_mesh("G0002", "LF1")
+    u0 = mesh.initialize(params, case.freestream)
+    args = ([mesh] * 3, [params] * 3, [u0] * 3)
+    assert AT.pick_few_shape(*args, precision=32, tile=64, seconds=0.02) == (0, 0, {})
+    assert AT.pick_few_slots(*args, precision=32, tile=64, seconds=0.02) == (0, {})
 
 
 def test_refill_and_release_keep_neighbours_bitwise():

@@ -73,6 +73,17 @@ def test_autotuner_few_slot_threshold():
     assert AT.choose_few({}) == 0
 
 
+def test_autotuner_few_slot_shape():
+    # The spread that beats the arena's own up to the most slots (the measured shape), or of two alike
+    # the faster one.
+    assert AT.choose_few_shape({2: {1: 66.2, 2: 61.4, 3: 57.5}, 8: {1: 69.3, 2: 64.5, 3: 72.3},
+                                16: {1: 82.6, 2: 77.4, 3: 113.6}, 32: {1: 101.4, 2: 117.1, 3: 166.8}}) == (16, 2)
+    assert AT.choose_few_shape({2: {1: 61.0, 2: 55.0, 3: 47.0}, 16: {1: 80.0, 2: 76.0, 3: 79.0}}) == (16, 3)
+    assert AT.choose_few_shape({2: {1: 61.0, 2: 55.0, 3: 56.0}, 8: {1: 70.0, 2: 71.0, 3: 65.0}}) == (8, 3)
+    assert AT.choose_few_shape({2: {2: 55.0, 3: 56.0}, 8: {2: 71.0, 3: 65.0}}) == (0, 0)
+    assert AT.choose_few_shape({}) == (0, 0)
+
+
 def test_autotuner_keeps_the_larger_tile_within_the_tie_margin():
     # A clear winner is kept whatever its size.
     assert AT.choose({64: 1.00e-3, 128: 1.10e-3, 256: 1.20e-3}) == 64
