@@ -629,6 +629,10 @@ int amr_batch_monitor(amr_batch* b, const int32_t* mask, const double* frames, c
                err, err_len, "AMR control D2H") ||
       !checked(b->arena->read_monitor(&cells, &walls, b->stream), err, err_len, "AMR monitor D2H"))
     return 1;
+  // The evaluation leaves the smallest local steps of the masked slots in their gather lines, which are
+  // otherwise empty between trials.  They stay there: the slot's next trial gathers those of the same
+  // accepted state (the base pass runs again, r0_valid 0), and whatever changes that state (admission)
+  // leaves the slot finished until the next targets, which clear the lines.
   std::vector<Control> restore = saved;
   for (int m = 0; m < n; ++m) {
     if (!use[m]) continue;
