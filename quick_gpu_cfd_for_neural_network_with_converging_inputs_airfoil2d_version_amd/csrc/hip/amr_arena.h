@@ -51,6 +51,7 @@ struct GatherLine {
 };
 static_assert(sizeof(GatherLine) == 128, "GatherLine layout");
 constexpr int kGatherLines = 32;
+constexpr size_t kGatherBytes = kGatherLines * sizeof(GatherLine);  // of a slot
 constexpr int kOneLineTiles = 160;
 __host__ __device__ constexpr int gather_lines(int tiles) { return tiles <= kOneLineTiles ? 1 : kGatherLines; }
 

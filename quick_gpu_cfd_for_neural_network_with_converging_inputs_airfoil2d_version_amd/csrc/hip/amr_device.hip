@@ -195,7 +195,7 @@ SlabPlan plan_slab(const Totals& t, int nv) {
                arr(4, t.groups) + arr(sizeof(T), t.groups) + arr(4, t.members) + arr(8, t.cell_blocks) +
                2 * arr(4, t.walls) + 4 * arr(sizeof(T), t.walls) + 2 * arr(8, t.walls);
   p.control = arr(sizeof(Control), t.meshes) + arr(sizeof(double), t.meshes) + arr(sizeof(long long), t.meshes) +
-              arr(6 * sizeof(double), t.meshes) + arr(sizeof(GatherLine) * kGatherLines, t.meshes);
+              arr(6 * sizeof(double), t.meshes) + arr(kGatherBytes, t.meshes);
   p.cplane = arr(sizeof(T), t.cells);
   p.dplane = arr(sizeof(double), t.cells);
   p.vec4 = arr(4 * sizeof(T), t.cells);
@@ -792,9 +792,10 @@ class DeviceArena final : public Arena {
         static_cast<size_t>(lds_max))
       return "AMR tile needs more LDS per block than the device provides";
     if (external_) {
+      // (The figures leave out the gather lines, for which the caller's memory has room of its own.)
       if (slab_bytes_ > external_bytes_)
-        return "AMR arena needs " + std::to_string(slab_bytes_) + " bytes; the device scratch holds " +
-               std::to_string(external_bytes_);
+        return "AMR arena needs " + std::to_string(slab_bytes_ - nm * kGatherBytes) +
+               " bytes; the device scratch holds " + std::to_string(external_bytes_ - nm * kGatherBytes);
       base = static_cast<char*>(external_);
     } else {
       if (hipMalloc(reinterpret_cast<void**>(&base), slab_bytes_) != hipSuccess) return "AMR hipMalloc of the arena failed";
@@ -851,7 +852,7 @@ class DeviceArena final : public Arena {
     a.mon_frame = frames_;
     offset += align256(nm * 6 * sizeof(double));
     a.gather = reinterpret_cast<GatherLine*>(base + offset);
-    offset += align256(nm * kGatherLines * sizeof(GatherLine));
+    offset += align256(nm * kGatherBytes);
     const size_t tables_end = offset;
     const auto dplanes = [&](int count) {
       double* p = reinterpret_cast<double*>(base + offset);

@@ -474,7 +474,9 @@ namespace {
 // (an LF2 mesh takes 8.5 MiB, a level-7 mesh 26 MiB) or twice that in FP32.
 constexpr size_t kScratchBytes = size_t(64) << 20;
 constexpr int kMaxDevices = 64;
-__device__ __align__(256) unsigned char scratch[kScratchBytes];
+// (The slot's gather lines, which came later, have their room beside it: they refuse no mesh.)
+constexpr size_t kScratchSize = kScratchBytes + hipamr::kGatherBytes;
+__device__ __align__(256) unsigned char scratch[kScratchSize];
 
 // Device address of `scratch` on each device (its host-side name is not a device address), and
 // one lock per device: calls from threads of this process on one device take turns, since each
@@ -516,7 +518,7 @@ extern "C" int amr_hip_run_noalloc(const amr_mesh_view* mesh, const amr_params* 
   // The same launch tile as a session of this mesh, so the two give the same bits.
   const int tile = mesh->n_cells < 200000 ? 64 : 256;
   std::unique_ptr<Arena> arena =
-      hipamr::make_arena({in}, precision, tile, stream, &message, scratch_ptr[device], kScratchBytes);
+      hipamr::make_arena({in}, precision, tile, stream, &message, scratch_ptr[device], kScratchSize);
   if (!arena) return fail(err, err_len, message);
   Control host{};
   hipamr::launch_target(arena->control(), arena->gather_lines(), 1, tend, maxsteps, nullptr, nullptr, stream);

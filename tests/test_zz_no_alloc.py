@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import _native as N
+from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd import batch as B
 from quick_gpu_cfd_for_neural_network_with_converging_inputs_airfoil2d_version_amd.session import BackendError, Session
 
 from .common import LAMINAR, case_mesh
@@ -70,3 +71,14 @@ def test_noalloc_fatal_and_limits():
     status, _, _, message = run_noalloc(big, bparams, big.initialize(bparams, case.freestream), 0.01, 64)
     print(message, flush=True)
     assert status == 1 and "the device scratch holds 67108864" in message
+
+
+def test_gather_lines_take_no_mesh_room():
+    """The 64 MiB are a mesh's own: the 32 gather lines of 128 bytes of its slot are not counted against
+    them, so that every mesh that fitted before there were any still does."""
+    case, big, bparams = case_mesh("G0001", "L8")
+    _, _, _, message = run_noalloc(big, bparams, big.initialize(bparams, case.freestream), 0.01, 64)
+    cap, features = B.capacity(big)
+    arena = B.arena_bytes([cap], features, precision=64, tile=64)
+    print(message, "arena of one slot", arena, flush=True)
+    assert f"needs {arena - 32 * 128} bytes" in message
