@@ -6,7 +6,7 @@ namespace hipamr {
 
 void launch_target(Control* ctrl, GatherLine* gather, int n, double target, long long maxsteps, const double* targets,
                    const long long* maxsteps_each, hipStream_t s) {
-  hipLaunchKernelGGL(k_target, dim3(blocks_of(n, 256)), dim3(256), 0, s, ctrl, gather, n, target, maxsteps, targets,
+  hipLaunchKernelGGL(k_target, dim3(blocks_of(n * kGatherLines, 256)), dim3(256), 0, s, ctrl, gather, n, target, maxsteps, targets,
                      maxsteps_each);
 }
 
