@@ -1377,8 +1377,7 @@ struct ugrid_session {
   std::vector<double> mco;   // host copy of the reference Mach numbers
   Control* host_ctrl = nullptr;  // pinned mirror of the control record
   hipStream_t stream = nullptr;
-  hipGraphExec_t exec = nullptr;      // trials, or backward-Euler rounds of kUpdates updates
-  hipGraphExec_t exec_one = nullptr;  // backward-Euler rounds of one update
+  hipGraphExec_t exec = nullptr;  // trials, or backward-Euler rounds of kUpdates updates
   std::vector<void*> owned;
 };
 
@@ -1410,8 +1409,7 @@ bool device_alloc(ugrid_session* s, T** p, size_t count, char* err, size_t len) 
 
 void release(ugrid_session* s) {
   if (!s) return;
-  for (hipGraphExec_t e : {s->exec, s->exec_one})
-    if (e) (void)hipGraphExecDestroy(e);
+  if (s->exec) (void)hipGraphExecDestroy(s->exec);
   for (void* p : s->owned) (void)hipFree(p);
   if (s->host_ctrl) (void)hipHostFree(s->host_ctrl);
   if (s->stream) (void)hipStreamDestroy(s->stream);
@@ -1507,8 +1505,8 @@ void launch_stage_srd(ugrid_session* s, hipStream_t stream) {
 // pays the three opening kernels once in eight updates, and at most a round less one of empty updates
 // at its end.  A step that needs kFewChecks updates or fewer (a nearly steady flow) wastes less in
 // rounds of one: 3 launches for each update but the first instead of 2 for each one missing of eight.
-// One case of 64 x 64 whose steps converge at their first check takes 45 us a step in long rounds and 24
-// in rounds of one, 8 cases of 256 x 256 99 and 59.  The host chooses by the updates a step of the last
+// One case of 64 x 64 whose steps converge at their first check takes 45 us a step in long rounds and 27
+// in rounds of one, 8 cases of 256 x 256 98 and 59.  The host chooses by the updates a step of the last
 // replay.
 constexpr int kUpdates = 8;
 constexpr int kFewChecks = 3;
@@ -1536,13 +1534,14 @@ int launch_trial(ugrid_session* s, hipStream_t stream) {
   return 4;
 }
 
-// `count` trials, or backward-Euler rounds of `updates` updates, as a graph.
-bool build_graph(ugrid_session* s, int count, int updates, hipGraphExec_t* exec, char* err, size_t len) {
+// `count` trials, or backward-Euler rounds, as a graph.
+bool build_graph(ugrid_session* s, int count, char* err, size_t len) {
   hipGraph_t graph = nullptr;
   if (!ok(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal), err, len, "begin capture")) return false;
   for (int k = 0; k < count; ++k) {
+constexpr int kShortRounds = 8;  // rounds of one update between polls
     if (s->par.time_integrator == 1)
-      launch_be_round(s, s->stream, updates);
+      launch_be_round(s, s->stream, kUpdates);
     else
       launch_trial(s, s->stream);
   }
@@ -1552,7 +1551,7 @@ bool build_graph(ugrid_session* s, int count, int updates, hipGraphExec_t* exec,
     if (graph) (void)hipGraphDestroy(graph);
     return false;
   }
-  const hipError_t inst = hipGraphInstantiate(exec, graph, nullptr, nullptr, 0);
+  const hipError_t inst = hipGraphInstantiate(&s->exec, graph, nullptr, nullptr, 0);
   (void)hipGraphDestroy(graph);
   return ok(inst, err, len, "graph instantiate");
 }
@@ -1858,8 +1857,7 @@ extern "C" int ugrid_create(const ugrid_setup* setup, const double* u, uint64_t 
   }
   const int trials = g.nx * static_cast<long long>(g.ny) * g.ncase >= (1 << 22) ? 4 : 16;
   const bool implicit = p.time_integrator == 1;
-  if (!build_graph(s, implicit ? trials / 4 : trials, kUpdates, &s->exec, err, err_len) ||
-      (implicit && !build_graph(s, trials / 2, 1, &s->exec_one, err, err_len))) {
+  if (!build_graph(s, implicit ? trials / 4 : trials, err, err_len)) {
     release(s);
     return 3;
   }
@@ -1912,19 +1910,21 @@ extern "C" int ugrid_run(ugrid_session* s, double tend, int64_t maxsteps, ugrid_
     if (now == progress) return fail(err, err_len, "ugrid_run: device step control made no progress");
     const bool first = progress == -1;
     progress = now;
-    hipGraphExec_t exec = s->exec;
     if (implicit) {
       const long long made = s->host_ctrl->nsteps - steps, tries = s->host_ctrl->checks + s->host_ctrl->iretries - used;
       steps += made;
       used += tries;
-      if (first) {
-        launch_be_round(s, s->stream, kUpdates);
+      const bool few = !first && made > 0 && tries <= kFewChecks * made;
+      if (first || few) {
+        // (Launched directly: a second graph would take longer to make than short runs take.)
+        const long long left = s->host_ctrl->maxsteps - s->host_ctrl->steps;
+        const int rounds = few ? static_cast<int>(std::clamp<long long>(left, 1, kShortRounds)) : 1;
+        for (int k = 0; k < rounds; ++k) launch_be_round(s, s->stream, few ? 1 : kUpdates);
         if (!ok(hipGetLastError(), err, err_len, "round launch")) return 3;
         continue;
       }
-      if (made > 0 && tries <= kFewChecks * made) exec = s->exec_one;
     }
-    if (!ok(hipGraphLaunch(exec, s->stream), err, err_len, "trial graph")) return 3;
+    if (!ok(hipGraphLaunch(s->exec, s->stream), err, err_len, "trial graph")) return 3;
   }
   const Control& c = *s->host_ctrl;
   if (meta) {
