@@ -1510,6 +1510,7 @@ void launch_stage_srd(ugrid_session* s, hipStream_t stream) {
 // replay.
 constexpr int kUpdates = 8;
 constexpr int kFewChecks = 3;
+constexpr int kShortRounds = 8;  // rounds of one update between polls
 int launch_be_round(ugrid_session* s, hipStream_t stream, int updates) {
   const Grid& g = s->g;
   const long long inner = static_cast<long long>(g.nx) * g.ny;
@@ -1539,7 +1540,6 @@ bool build_graph(ugrid_session* s, int count, char* err, size_t len) {
   hipGraph_t graph = nullptr;
   if (!ok(hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal), err, len, "begin capture")) return false;
   for (int k = 0; k < count; ++k) {
-constexpr int kShortRounds = 8;  // rounds of one update between polls
     if (s->par.time_integrator == 1)
       launch_be_round(s, s->stream, kUpdates);
     else
