@@ -264,15 +264,32 @@ class Solver2D:
         return DeviceSession(self)
 
 
+_LARGE = 1 << 22  # bytes from which a state is worth four threads
+
+
+def _in_parts(size: int, work) -> None:
+    """work(slice) on four quarters of range(size), a thread each."""
+    with ThreadPoolExecutor(4) as pool:
+        list(pool.map(lambda k: work(slice(size * k // 4, size * (k + 1) // 4)), range(4)))
+
+
 def _copy_state(dst: np.ndarray, src: np.ndarray) -> None:
     """dst[:] = src; a large state in four threads (270 MB: 9.1 -> 3.2 ms)."""
-    if src.nbytes < (1 << 22) or dst.dtype != src.dtype or not (dst.flags.c_contiguous and src.flags.c_contiguous):
+    if src.nbytes < _LARGE or dst.dtype != src.dtype or not (dst.flags.c_contiguous and src.flags.c_contiguous):
         dst[:] = src
         return
     flat, source = dst.reshape(-1), src.reshape(-1)
-    cuts = [src.size * k // 4 for k in range(5)]
-    with ThreadPoolExecutor(4) as pool:
-        list(pool.map(lambda k: np.copyto(flat[cuts[k]:cuts[k + 1]], source[cuts[k]:cuts[k + 1]]), range(4)))
+    _in_parts(src.size, lambda part: np.copyto(flat[part], source[part]))
+
+
+def _touched(shape) -> np.ndarray:
+    """An array whose pages are in memory, so that the first download into it does not wait for them one by
+    one (270 MB: a first pull of 37 -> 31 ms)."""
+    a = np.empty(shape)
+    if a.nbytes >= _LARGE:
+        flat = a.reshape(-1)
+        _in_parts(a.size, lambda part: np.copyto(flat[part][::512], 0.0))
+    return a
 
 
 class DeviceSession:
@@ -306,7 +323,7 @@ class DeviceSession:
         err = N.err_buffer()
         # Into buffers of the session first: a download that fails leaves the solver as it was.
         if self._staging is None or self._staging.shape != s.U.shape:
-            self._staging = np.empty(s.U.shape)
+            self._staging = _touched(s.U.shape)
         u = self._staging
         t = np.empty(s.ncase)
         dt = np.empty(s.ncase)
