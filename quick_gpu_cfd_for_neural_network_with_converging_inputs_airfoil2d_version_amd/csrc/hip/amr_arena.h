@@ -41,7 +41,10 @@ static_assert(sizeof(Control) == 128, "Control layout");
 // take about 9 ns each and hold up reads of their cache line, so in the control records, 112 bytes
 // apart, they delayed every block of the slot and its neighbours: one level-8 mesh (1640 tiles) 124 ->
 // 98 us a trial in FP64 and 90 -> 62 in FP32, 16 meshes of mixed levels 99 -> 91, 8 LF2 meshes at
-// tile 64 71 -> 64.  One LF2 mesh (150 tiles) would lose 0.8 us to the second round of atomics.
+// tile 64 71 -> 64.  A small slot would lose to the second round of atomics.  One line against 32, us a
+// trial of one mesh, FP32 / FP64: 75 tiles 46.6 : 47.8 / 53.6 : 54.6, 115 50.7 : 51.6 / 62.8 : 64.0, 149
+// 44.4 : 45.3 / 51.2 : 52.1, 230 46.4 : 45.8 / 55.0 : 55.1, 409 66.3 : 64.4 / 102.4 : 102.3, 459 51.0 :
+// 45.7 / 58.3 : 55.4, 818 73.3 : 64.0 / 111 : 101; the line lies between the last loss and the first gain.
 struct GatherLine {
   unsigned long long dt_min;    // bit pattern of the minimum local dt of the base pass
   // Blocks of the last stage pass that have finished this trial (low 32 bits) and how many of

@@ -842,7 +842,9 @@ __device__ __forceinline__ void arrive_and_commit(Control* c, GatherLine* line, 
 // (72 VGPRs, 4 and 6 spilled; LDS for 14 blocks per CU).
 // On 256 LF2 meshes: base flux 187 -> 177 us, stage flux 188 -> 181 us against the unbounded
 // kernels; 8 waves (64 VGPRs) spills 11-14 and is slower.  FP64: 3 waves (157-167 VGPRs, no spill;
-// see late_gradients).
+// see late_gradients).  On 64 LF2 meshes at tile 128 the FP64 passes hold 1.9 (base: LDS admits 2.5) and
+// 2.2 waves per SIMD, VALU busy 43 and 39% of the time at 2.3 and 3.5 TB/s: what bounds them is the
+// latency of loads and of dependent FP64 operations that so few waves cover.
 // SPREAD threads per cell (1 to 3): a tile's face items are spread over SPREAD * tile threads,
 // the cell work stays on the first tile of them (a separate instantiation, so that the one-thread
 // kernel keeps its registers).  A tile touches 2.2 - 2.7 faces per cell, so three threads per cell

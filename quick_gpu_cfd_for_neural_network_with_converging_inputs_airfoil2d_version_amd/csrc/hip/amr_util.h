@@ -38,8 +38,6 @@ inline hipError_t copy_sync(void* dst, const void* src, size_t bytes, hipMemcpyK
   return e != hipSuccess ? e : hipStreamSynchronize(stream);
 }
 
-constexpr unsigned long long kInfBitsHost = 0x7ff0000000000000ull;
-
 // Records a hipEvent pair around every kernel launch on a stream.
 struct EventHook final : LaunchHook {
   hipStream_t stream;

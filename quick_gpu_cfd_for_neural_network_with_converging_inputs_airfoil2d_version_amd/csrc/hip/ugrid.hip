@@ -53,7 +53,8 @@ constexpr int kMaxRetries = 12;
 constexpr int kDecide = 1024;      // threads of the decision kernels that reduce the strips' partials
 // Cases up to which strips store their maxima for the decision kernel instead of one 64-bit
 // atomicMax per strip on the case's word: device-scope atomics on one word take about 9 ns each
-// (4 cases of 400 x 311, 2184 strips: last stage 44 us, of which 20 us were its atomics).  With more
+// (4 cases of 400 x 311, 2184 strips: last stage 44 us, of which 20 us were its atomics).  The decision
+// takes longer for it (8 cases of 1024 x 1024, 6120 strips: 5.6 -> 9.6 us of a 590 us step).  With more
 // cases the words are many and the reduction's table would not fit LDS.
 constexpr int kPartCases = 1024;
 // Steps a first-stage pre-check tries on a cut grid (the body bench needs about six halvings a step).
@@ -553,11 +554,13 @@ __device__ void commit(const Grid& g, unsigned long long* s_max) {
 __device__ __forceinline__ void load_row(const double* p, size_t plane, double (&c)[4]) {
   for (int v = 0; v < 4; ++v) c[v] = p[v * plane];
 }
-// Bound by FP64 instruction issue (about 480 VALU instructions a cell, 930 with every quotient a full
-// division and both sides' sound speeds, energies and enthalpies formed at every face) and by the
-// latency of its row's loads: the next row's state is loaded while this one is evaluated, the base
-// state of the row to update before the y fluxes.  That takes 136 VGPRs (150-160 on a cut grid) and
-// three waves per SIMD; four waves (128 VGPRs) spill nothing but the loads' lead: 8 cases of
+// Bound by FP64 instruction issue (about 450 VALU instructions a cell of a row, halos included, 875 with
+// every quotient a full division and both sides' sound speeds, energies and enthalpies formed at every
+// face; VALU busy 75 / 66 / 68% of the three stages on 16 cases of 1024 x 1024), in stages 2 and 3 also by
+// memory (4.5-4.7 TB/s, 78% of the best copy), and by the latency of its row's loads: the next row's state is loaded while this one is evaluated, the base
+// state of the row to update before the y fluxes.  That takes 124-146 VGPRs (RK stages; 146-166 on a cut
+// grid), 130-173 in the pseudo update, and three waves per SIMD (168 VGPRs; the cut grid's HLLC pseudo
+// update, 173, has two); four waves (128 VGPRs) spill nothing but the loads' lead: 8 cases of
 // 1024 x 1024, HLLC, stages 336 / 347 / 378 us before, 218 / 276 / 294 with four waves and no
 // prefetch, 202 / 230 / 244 with it.
 template <int MODE, bool CUT, bool AUSM>
@@ -617,7 +620,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(CUT ? 
     double q0 = 0, q1 = 0, q2 = 0, q3 = 0;  // conserved state of the owned cell of the previous row
     unsigned code_prev = 0;                  // cut grids: code of the lane's cell of the previous row
     const bool in_x = i >= 0 && i <= g.nx;   // the lane's west x face is a grid face
-    bool flip_v = false, flip_next = false;
+    bool flip_v = false;
     int jc = map_axis(j0 - 1, g.ny, g.bc[2], g.bc[3], &flip_v);
     double next[4];
     load_row(in + case_base + static_cast<size_t>(jc + kGhosts) * g.mx, plane, next);
@@ -1699,11 +1702,13 @@ bool upload_cut(ugrid_session* s, const ugrid_cut_view& c, const double* dx, con
 
 // Rows per strip.  A strip of r rows costs its wave about r + 1 row times (the halo row's
 // primitives and y flux), and a CU that holds n = 1, 2, 3 blocks (three is what the registers admit)
-// takes kRowTime[n] microseconds a row, as fitted to launches of 1 to 64 rows on five grids.  Long
+// takes kRowTime[n] microseconds a row, as fitted to launches of 1 to 64 rows on five grids (a cut grid's
+// HLLC pseudo update has two blocks in a CU; its strips are chosen as for three).  Long
 // strips waste least on the halo, short ones spread a small grid over the chip, and a launch that
 // leaves its last round of blocks nearly empty pays for a whole one: the count with the least estimate
-// is chosen.  Against 32 rows, halved down to 4 while a CU held fewer than 16 waves: 8 cases of
-// 1024 x 1024 682 us a step at 32 rows and 594 at 47 (2992 waves of 3072 slots), 3 of 200 x 131
+// is chosen, of counts that tie the smallest.  Against 32 rows, halved down to 4 while a CU held fewer
+// than 16 waves: 8 cases of 1024 x 1024 682 us a step at 32 rows, 587 at the 23 that it takes (6120
+// strips, two rounds of three blocks a CU) and 596 at 47 (2992, one round; the same estimate), 3 of 200 x 131
 // 39.4 us at 4 rows and 27.6 at 1, 4 of 400 x 311 70.6 us at 4 and 62.3 at 3.
 int choose_rows(int nx, int ny, int ncase, bool cut) {
   constexpr int kCus = 256, kResident = 3, kLongest = 64;
