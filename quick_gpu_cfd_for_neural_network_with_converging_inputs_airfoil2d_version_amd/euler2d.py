@@ -264,7 +264,9 @@ class Solver2D:
         return DeviceSession(self)
 
 
-_LARGE = 1 << 22  # bytes from which a state is worth four threads
+# Bytes from which a state is copied by four threads: 17 MB take 0.23 ms in one and 0.30 in four, 34 MB
+# 1.03 and 0.52.
+_LARGE = 1 << 25
 
 
 def _in_parts(size: int, work) -> None:

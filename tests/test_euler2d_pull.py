@@ -54,7 +54,7 @@ def test_failed_download_leaves_the_solver(lib):
 
 
 @pytest.mark.parametrize("layout", ["own", "float32", "strided"])
-@pytest.mark.parametrize("nx, ny, cases", [(1, 1, 1), (357, 363, 1), (358, 363, 1), (401, 333, 3)])
+@pytest.mark.parametrize("nx, ny, cases", [(1, 1, 1), (1020, 1019, 1), (1020, 1020, 1), (637, 501, 4)])
 def test_whole_state_lands(nx, ny, cases, layout):  # below, at and above the size that is copied in parts
     s, d = session(nx, ny, cases, Library())
     if layout == "float32":
