@@ -839,7 +839,7 @@ __device__ __forceinline__ void arrive_and_commit(Control* c, GatherLine* line, 
 // FP32 register budget: 5 waves per SIMD in the base pass (89 VGPRs, no spill; its LDS admits
 // 11 blocks of two waves per CU, 5.5 waves per SIMD, so a 6-wave bound, which spilled, bought no
 // occupancy: base flux 151 -> 141 us with the batched entries below) and 7 in the stage passes
-// (72 VGPRs, 4 and 6 spilled; LDS for 14 blocks per CU).
+// (72 VGPRs, no spill; LDS for 14 blocks per CU).
 // On 256 LF2 meshes: base flux 187 -> 177 us, stage flux 188 -> 181 us against the unbounded
 // kernels; 8 waves (64 VGPRs) spills 11-14 and is slower.  FP64: 3 waves (157-167 VGPRs, no spill;
 // see late_gradients).  On 64 LF2 meshes at tile 128 the FP64 passes hold 1.9 (base: LDS admits 2.5) and

@@ -557,7 +557,7 @@ __device__ __forceinline__ void load_row(const double* p, size_t plane, double (
 // Bound by FP64 instruction issue (about 450 VALU instructions a cell of a row, halos included, 875 with
 // every quotient a full division and both sides' sound speeds, energies and enthalpies formed at every
 // face; VALU busy 75 / 66 / 68% of the three stages on 16 cases of 1024 x 1024), in stages 2 and 3 also by
-// memory (4.5-4.7 TB/s, 78% of the best copy), and by the latency of its row's loads: the next row's state is loaded while this one is evaluated, the base
+// memory (4.5-4.6 TB/s, three quarters of the best copy), and by the latency of its row's loads: the next row's state is loaded while this one is evaluated, the base
 // state of the row to update before the y fluxes.  That takes 124-146 VGPRs (RK stages; 146-166 on a cut
 // grid), 130-173 in the pseudo update, and three waves per SIMD (168 VGPRs; the cut grid's HLLC pseudo
 // update, 173, has two); four waves (128 VGPRs) spill nothing but the loads' lead: 8 cases of
