@@ -1389,6 +1389,7 @@ struct ugrid_session {
   Control* host_ctrl = nullptr;  // pinned mirror of the control record
   hipStream_t stream = nullptr;
   hipGraphExec_t exec = nullptr;  // trials, or backward-Euler rounds of kUpdates updates
+  bool few_checks = false;  // backward Euler: the last replay's steps needed kFewChecks updates or fewer
   std::vector<void*> owned;
 };
 
@@ -1537,8 +1538,8 @@ void launch_stage_srd(ugrid_session* s, hipStream_t stream) {
 // at its end.  A step that needs kFewChecks updates or fewer (a nearly steady flow) wastes less in
 // rounds of one: 3 launches for each update but the first instead of 2 for each one missing of eight.
 // One case of 64 x 64 whose steps converge at their first check takes 45 us a step in long rounds and 27
-// in rounds of one, 8 cases of 256 x 256 98 and 59.  The host chooses by the updates a step of the last
-// replay.
+// in rounds of one, 8 cases of 256 x 256 98 and 59.  The host chooses by the updates a step of the
+// session's last replay.
 constexpr int kUpdates = 8;
 constexpr int kFewChecks = 3;
 constexpr int kShortRounds = 8;  // rounds of one update between polls
@@ -1937,32 +1938,27 @@ extern "C" int ugrid_run(ugrid_session* s, double tend, int64_t maxsteps, ugrid_
   // phase change), so it must move the event count; a replay that does not is reported, not
   // waited on.
   long long progress = -1;
-  // Backward Euler: steps, and update kernels that they used, up to the last poll; the first round of a
-  // run is launched by itself, and those after it by what it showed.
-  long long steps = 0, used = 0;
+  long long steps = 0, used = 0;  // backward Euler: steps, and update kernels that they used, up to the last poll
   for (;;) {
     if (!ok(hipMemcpyAsync(s->host_ctrl, g.ctrl, sizeof(Control), hipMemcpyDeviceToHost, s->stream), err, err_len,
             "control copy") ||
         !ok(hipStreamSynchronize(s->stream), err, err_len, "trial"))
       return 3;
+    const long long made = s->host_ctrl->nsteps - steps, tries = s->host_ctrl->checks + s->host_ctrl->iretries - used;
+    steps += made;
+    used += tries;
+    if (implicit && progress != -1) s->few_checks = made > 0 && tries <= kFewChecks * made;
     if (s->host_ctrl->status != RUNNING) break;
     const long long now = s->host_ctrl->events;
     if (now == progress) return fail(err, err_len, "ugrid_run: device step control made no progress");
-    const bool first = progress == -1;
     progress = now;
-    if (implicit) {
-      const long long made = s->host_ctrl->nsteps - steps, tries = s->host_ctrl->checks + s->host_ctrl->iretries - used;
-      steps += made;
-      used += tries;
-      const bool few = !first && made > 0 && tries <= kFewChecks * made;
-      if (first || few) {
-        // (Launched directly: a second graph would take longer to make than short runs take.)
-        const long long left = s->host_ctrl->maxsteps - s->host_ctrl->steps;
-        const int rounds = few ? static_cast<int>(std::clamp<long long>(left, 1, kShortRounds)) : 1;
-        for (int k = 0; k < rounds; ++k) launch_be_round(s, s->stream, few ? 1 : kUpdates);
-        if (!ok(hipGetLastError(), err, err_len, "round launch")) return 3;
-        continue;
-      }
+    if (s->few_checks) {
+      // (Launched directly: a second graph would take longer to make than short runs take.)
+      const long long left = s->host_ctrl->maxsteps - s->host_ctrl->steps;
+      const long long rounds = std::clamp<long long>(left, 1, kShortRounds);
+      for (long long k = 0; k < rounds; ++k) launch_be_round(s, s->stream, 1);
+      if (!ok(hipGetLastError(), err, err_len, "round launch")) return 3;
+      continue;
     }
     if (!ok(hipGraphLaunch(s->exec, s->stream), err, err_len, "trial graph")) return 3;
   }

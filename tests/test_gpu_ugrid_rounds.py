@@ -46,7 +46,7 @@ def test_steps_of_few_and_many_updates(cfl, tol, per_step, runs):
 
 def test_step_that_converges_at_once_is_short():
     """A uniform state's step is five dependent launches, an SSP-RK3 step four (stages that march three
-    rows as the update does): 26 against 22 us on one case of 64 x 64, 45 where a step's round holds
+    rows as the update does): 27 against 22 us on one case of 64 x 64, 45 where a step's round holds
     eight updates."""
     best = {}
     for integrator in (E.TIME_BACKWARD_EULER, E.TIME_SSP_RK3):
